@@ -217,6 +217,13 @@ int vx_gemm_f32_route(const vx_mview* out, const vx_cview* lhs,
  * point has none, so they are computed with x kept in f32 (the
  * VX_GEMV_X_F32 kernels); vx_gemv_q_ws with a caller workspace keeps the
  * int8 split there (the fused and the two-launch route give the same bits).
+ * Many columns: with x kept in f32 and B > 4, and with a workspace and B > 16
+ * where that is the faster route, the product runs on the bf16 matrix cores
+ * with x as the sum of bf16 terms: three, which hold a float exactly, where x
+ * is kept in f32; two, |error| <= 2^-16 |x| per element (closer than the int8
+ * split), with a workspace. Products with the whole-number weights are exact,
+ * sums and scaling f32. A non-finite x reaches its own column only, as on the
+ * other routes.
  * Empty shapes: K = 0 writes y = 0 (as vx_gemm_f32 with K = 0); M = 0 or
  * B = 0 returns VX_OK and launches nothing. The same holds for _ex, _ws
  * and _noalloc; vx_gemv_q_xq also returns VX_OK for M = 0 or B = 0 but
@@ -248,8 +255,8 @@ int vx_gemv_q_ex(vx_ctx ctx, vx_stream stream, const vx_mview* y,
  * (src/linalg/gemm.rs:47-56): per-caller mutable state kept outside the
  * (immutable) context. Where a batched call needs its activation split in
  * memory (see vx_gemv_q), x is split into `workspace` by the vx_quantize_x
- * kernel and the GEMV reads it (two launches on `stream`); elsewhere the
- * workspace is not touched. workspace: device memory, 16-byte aligned, at
+ * kernel and the GEMV reads it (two launches on `stream`); elsewhere, many
+ * columns (vx_gemv_q) among it, the workspace is not touched. workspace: device memory, 16-byte aligned, at
  * least vx_gemv_q_ws_size(...) bytes (a smaller non-NULL workspace is
  * VX_ERR_INVALID; NULL behaves as vx_gemv_q_ex). The library never
  * allocates, frees or retains it; its contents need not start at zero.

@@ -13,7 +13,8 @@
 //   * the decoded dot uses one byte->float convert and one FMA per
 //     weight; x for the unit stays in 64 VGPRs across the R rows;
 //   * partial sums are reduced across the wave with xor shuffles.
-// Batch > 1 uses the same staging with exact per-weight decode and x read
+// Batches of 2..4 with x kept in f32 use the same staging with exact per-weight
+// decode (more columns: gemm_q.hip) and x read
 // from LDS per 8-weight group; lanes are split into 64/LPR row groups so
 // that NB * chunk fits the LDS budget.
 #include "vx_quant.hpp"
@@ -1085,8 +1086,6 @@ __device__ __forceinline__ vx_gemv_args vx_b1_args(const uint8_t* w, const float
     VX_GEMV_I8B1(QT, QN, 8)                                                                         \
     VX_GEMV_BN(QT, QN, 2, 2, 64)                                                                    \
     VX_GEMV_BN(QT, QN, 4, 2, 64)                                                                    \
-    VX_GEMV_BN(QT, QN, 8, 2, 32)                                                                    \
-    VX_GEMV_BN(QT, QN, 16, 2, 16)                                                                   \
     extern "C" __global__ __launch_bounds__(VX_WG) void vx_gemv_generic_##QN(vx_gemv_args a) {     \
         vx_args_fetch(a);                                                                           \
         vx_gemv_generic<QT>(a);                                                                     \
@@ -1163,46 +1162,6 @@ VX_READ_PROBE(VX_Q4_K, q4_k)
 // XI = 1). At the end of each tile the 16 waves' partial sums meet in LDS and
 // one thread per output adds them in slice order (deterministic), adding to
 // its own y of the previous passes when K takes several passes.
-
-// v_permlane{16,32}_swap results pass through empty asm: see vx_pin2.
-__device__ __forceinline__ void vx_swap32(uint32_t& x, uint32_t& y) {
-    vx_pin2(x, y);
-    const auto s = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-    x = s[0];
-    y = s[1];
-    vx_pin2(x, y);
-}
-__device__ __forceinline__ void vx_swap16(uint32_t& x, uint32_t& y) {
-    vx_pin2(x, y);
-    const auto s = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-    x = s[0];
-    y = s[1];
-    vx_pin2(x, y);
-}
-
-// 4 x 4 transpose across the 16-lane rows: on entry row u of r[k] holds
-// A[u][k]; on exit row g of r[k] holds A[k][g]. permlane32_swap(x, y)
-// exchanges rows 2, 3 of x with rows 0, 1 of y; permlane16_swap(x, y) rows
-// 1, 3 of x with rows 0, 2 of y.
-__device__ __forceinline__ void vx_t4(uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3) {
-    vx_swap32(r0, r2);  // r0 = [A00 A10 A02 A12], r2 = [A20 A30 A22 A32]
-    vx_swap32(r1, r3);  // r1 = [A01 A11 A03 A13], r3 = [A21 A31 A23 A33]
-    vx_swap16(r0, r1);  // r0 = [A00 A01 A02 A03], r1 = [A10 A11 A12 A13]
-    vx_swap16(r2, r3);  // r2 = [A20 A21 A22 A23], r3 = [A30 A31 A32 A33]
-}
-
-// Every row's value of v in every lane: o[u] = v of 16-lane row u.
-__device__ __forceinline__ void vx_gather4(uint32_t v, uint32_t (&o)[4]) {
-    uint32_t a = v, b = v;
-    vx_swap32(a, b);  // a = [v0 v1 v0 v1], b = [v2 v3 v2 v3]
-    uint32_t a2 = a, b2 = b;
-    vx_swap16(a, a2);  // a = [v0 v0 v0 v0], a2 = [v1 v1 v1 v1]
-    vx_swap16(b, b2);  // b = [v2 v2 v2 v2], b2 = [v3 v3 v3 v3]
-    o[0] = a;
-    o[1] = a2;
-    o[2] = b;
-    o[3] = b2;
-}
 
 // The weights of one item (8 blocks / sub-blocks of 32) in MFMA layout.
 template <int QT>

@@ -1,0 +1,55 @@
+// vx_bf16.hpp — f32 values as sums of bfloat16 terms, for the bf16 matrix
+// cores (no reference counterpart).
+//
+// A bf16 value has 8 significant bits and float's exponent range, so a float
+// is the sum of three bf16 terms exactly, and of two to within 2^-16 of its
+// magnitude. Products of two bf16 values are exact in f32, and the matrix
+// cores add them in f32: a contraction over three terms is an f32
+// contraction, at a rate of 1/3 (one operand split) of ~2.5 PFLOP/s against
+// the f32 matrix cores' 157 TFLOP/s.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// (a, b) rounded to nearest even, a in the low half.
+__device__ __forceinline__ uint32_t vx_pk_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+// The high halves of (a, b), a in the low half: both truncated to bf16.
+__device__ __forceinline__ uint32_t vx_pk_hi(uint32_t a, uint32_t b) {
+    return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+
+// v[0..8) as NT terms of packed bf16, largest first. The leading terms are
+// truncated (a rounded one could overflow to infinity for |v| near the
+// largest float; the remainder v - trunc(v) is exact either way). NT = 3: the
+// last term has at most 8 bits left, so the three add up to v exactly (down
+// to bf16's smallest subnormal, 2^-133). NT = 2: the last term is rounded,
+// error <= 2^-16 |v|. An infinity gives {inf, NaN, ..}, a NaN {NaN, ..}.
+template <int NT>
+__device__ __forceinline__ void vx_split8(const float (&v)[8], u32x4 (&t)[NT]) {
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = v[i];
+#pragma unroll
+    for (int k = 0; k < NT - 1; ++k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t a = __float_as_uint(r[2 * i]), b = __float_as_uint(r[2 * i + 1]);
+            t[k][i] = vx_pk_hi(a, b);
+            r[2 * i] -= __uint_as_float(a & 0xFFFF0000u);
+            r[2 * i + 1] -= __uint_as_float(b & 0xFFFF0000u);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        t[NT - 1][i] = NT == 3 ? vx_pk_hi(__float_as_uint(r[2 * i]), __float_as_uint(r[2 * i + 1]))
+                               : vx_pk_bf16(r[2 * i], r[2 * i + 1]);
+}

@@ -7,6 +7,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 // DPP controls used here (GFX9 encoding):
 //   0xB1  quad_perm [1,0,3,2]   lane i <- i ^ 1
@@ -93,4 +94,44 @@ __device__ __forceinline__ float vx_sum_rows4x4(float v0, float v1, float v2, fl
     unsigned t0 = t[0], t1 = t[1];
     vx_pin2(t0, t1);
     return __builtin_bit_cast(float, t0) + __builtin_bit_cast(float, t1);
+}
+
+// v_permlane{16,32}_swap with operands and results through empty asm (see vx_pin2).
+__device__ __forceinline__ void vx_swap32(uint32_t& x, uint32_t& y) {
+    vx_pin2(x, y);
+    const auto s = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = s[0];
+    y = s[1];
+    vx_pin2(x, y);
+}
+__device__ __forceinline__ void vx_swap16(uint32_t& x, uint32_t& y) {
+    vx_pin2(x, y);
+    const auto s = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    x = s[0];
+    y = s[1];
+    vx_pin2(x, y);
+}
+
+// 4 x 4 transpose across the 16-lane rows: on entry row u of r[k] holds
+// A[u][k]; on exit row g of r[k] holds A[k][g]. permlane32_swap(x, y)
+// exchanges rows 2, 3 of x with rows 0, 1 of y; permlane16_swap(x, y) rows
+// 1, 3 of x with rows 0, 2 of y.
+__device__ __forceinline__ void vx_t4(uint32_t& r0, uint32_t& r1, uint32_t& r2, uint32_t& r3) {
+    vx_swap32(r0, r2);  // r0 = [A00 A10 A02 A12], r2 = [A20 A30 A22 A32]
+    vx_swap32(r1, r3);  // r1 = [A01 A11 A03 A13], r3 = [A21 A31 A23 A33]
+    vx_swap16(r0, r1);  // r0 = [A00 A01 A02 A03], r1 = [A10 A11 A12 A13]
+    vx_swap16(r2, r3);  // r2 = [A20 A21 A22 A23], r3 = [A30 A31 A32 A33]
+}
+
+// Every row's value of v in every lane: o[u] = v of 16-lane row u.
+__device__ __forceinline__ void vx_gather4(uint32_t v, uint32_t (&o)[4]) {
+    uint32_t a = v, b = v;
+    vx_swap32(a, b);  // a = [v0 v1 v0 v1], b = [v2 v3 v2 v3]
+    uint32_t a2 = a, b2 = b;
+    vx_swap16(a, a2);  // a = [v0 v0 v0 v0], a2 = [v1 v1 v1 v1]
+    vx_swap16(b, b2);  // b = [v2 v2 v2 v2], b2 = [v3 v3 v3 v3]
+    o[0] = a;
+    o[1] = a2;
+    o[2] = b;
+    o[3] = b2;
 }

@@ -31,6 +31,8 @@ extern const unsigned char vx_co_copy[];
 extern const unsigned char vx_co_copy_end[];
 extern const unsigned char vx_co_quantize[];
 extern const unsigned char vx_co_quantize_end[];
+extern const unsigned char vx_co_gemm_q[];
+extern const unsigned char vx_co_gemm_q_end[];
 }
 
 namespace vx {
@@ -69,8 +71,8 @@ static const char* const kKernelNames[K_COUNT] = {
 #undef K
 };
 // The embedded code objects; every kernel name is unique across them.
-static const unsigned char* const kModules[] = {vx_co_gemm, vx_co_gemv_q, vx_co_copy, vx_co_quantize};
-constexpr int kNumModules = 4;
+static const unsigned char* const kModules[] = {vx_co_gemm, vx_co_gemv_q, vx_co_copy, vx_co_quantize, vx_co_gemm_q};
+constexpr int kNumModules = 5;
 constexpr int kModGemv = 1;  // the module holding vx_scratch
 
 }  // namespace vx
@@ -492,12 +494,10 @@ static int i8b1_kernel(uint32_t qt, int R) {
 }
 
 static int bn_kernel(uint32_t qt, int NB) {
-    static const int tab[3][4] = {
-        {K_vx_gemv_b2_q4_0_r2, K_vx_gemv_b4_q4_0_r2, K_vx_gemv_b8_q4_0_r2, K_vx_gemv_b16_q4_0_r2},
-        {K_vx_gemv_b2_q8_0_r2, K_vx_gemv_b4_q8_0_r2, K_vx_gemv_b8_q8_0_r2, K_vx_gemv_b16_q8_0_r2},
-        {K_vx_gemv_b2_q4_k_r2, K_vx_gemv_b4_q4_k_r2, K_vx_gemv_b8_q4_k_r2, K_vx_gemv_b16_q4_k_r2}};
-    const int ni = NB == 2 ? 0 : NB == 4 ? 1 : NB == 8 ? 2 : 3;
-    return tab[q_index(qt)][ni];
+    static const int tab[3][2] = {{K_vx_gemv_b2_q4_0_r2, K_vx_gemv_b4_q4_0_r2},
+                                  {K_vx_gemv_b2_q8_0_r2, K_vx_gemv_b4_q8_0_r2},
+                                  {K_vx_gemv_b2_q4_k_r2, K_vx_gemv_b4_q4_k_r2}};
+    return tab[q_index(qt)][NB == 2 ? 0 : 1];
 }
 
 // Persistent batch-1 kernel with f32 x (VX_GEMV_X_F32); xv: x contiguous
@@ -790,6 +790,84 @@ static int run_gemv_q_xq(vx_ctx ctx, vx_stream stream, const vx_mview* y, const 
     return launch_gemv_xq(ctx, stream, cy, w, q);
 }
 
+// ------------------------------------------------ many columns of x
+// Products with more columns of x than a GEMV launch takes run on the bf16
+// matrix cores (gemm_q.hip) with x as two bf16 terms (where x may be rounded)
+// or three (x exact). Four kernels: 32 x 16, 64 x 16 and 64 x 32 outputs per
+// workgroup with K split over its eight waves, and 256 x 128 tiles that share
+// the converted x through LDS. Which is fastest is a question of rounds: one
+// workgroup runs per CU, and a round takes about the same time per 32-block
+// of K however full it is. kGemmQ: measured nanoseconds of a round per
+// 32-block (K = 4096; 1024..32000 rows, 2..512 columns), Q4_0 / Q4_K and
+// Q8_0, two and three terms.
+static const double kGemmQ[2][2][4] = {{{95, 125, 178, 1100}, {105, 150, 205, 1300}},
+                                       {{98, 150, 205, 1490}, {112, 170, 235, 1710}}};
+static const uint32_t kGemmQRows[4] = {32, 64, 64, 256}, kGemmQCols[4] = {16, 16, 32, 128};
+
+static bool gemm_q_ok(const vx_qweight* w) { return xq_layout_ok(w) && w->cols <= (1u << 28); }
+
+// The kernel (index into kGemmQ's last dimension) for M x K times B columns
+// with nt terms, and its estimated time.
+static int gemm_q_choose(vx_ctx ctx, uint32_t qt, uint32_t M, uint32_t K, uint32_t B, int nt, double* us) {
+    int best = 0;
+    for (int c = 0; c < 4; ++c) {
+        const double wgs = std::ceil((double)M / kGemmQRows[c]) * std::ceil((double)B / kGemmQCols[c]);
+        const double t = std::ceil(wgs / ctx->num_cus) * (K / 32u) * kGemmQ[nt - 2][qt == VX_Q8_0][c] * 1e-3;
+        if (c == 0 || t < *us) best = c, *us = t;
+    }
+    return best;
+}
+
+// Estimated time of the route through the int8 split (vx_quantize_x, then a
+// launch per 16 columns, each streaming W): a launch costs about 4 us and its
+// bytes, 0.155 (Q4_0, Q4_K) or 0.19 us (Q8_0) per million weights, a fifth
+// more when K takes several passes, a fifth less with up to 8 columns
+// (measured as kGemmQ; 4096 x 4096 x 32 15 us, 11008 x 4096 x 64 42..55 us,
+// 4096 x 11008 x 64 52..64 us).
+static double gemv_xq_us(uint32_t qt, uint32_t M, uint32_t K, uint32_t B) {
+    const double one = (3.9 + (double)M * K * 1e-6 * (qt == VX_Q8_0 ? 0.19 : 0.155)) * (K > 4096u ? 1.2 : 1.0);
+    const uint32_t full = B / 16u, rem = B % 16u;
+    return 2.2 + one * full + (rem == 0u ? 0.0 : rem <= 8u ? 0.8 * one : one);
+}
+
+static int launch_gemm_q(vx_ctx ctx, vx_stream stream, const Canon& cy, const vx_qweight* w, const Canon& cx, uint32_t B,
+                         int nt, int cfg) {
+#define VX_GQ1(N) {K_vx_gemm_q_##N, K_vx_gemm_q_##N##_xs}
+#define VX_GQ(N) {VX_GQ1(N##_ks2x1), VX_GQ1(N##_ks4x1), VX_GQ1(N##_ks4x2), VX_GQ1(N##_256x128)}
+    static const int tab[3][2][4][2] = {{VX_GQ(q4_0_t2), VX_GQ(q4_0_t3)}, {VX_GQ(q8_0_t2), VX_GQ(q8_0_t3)},
+                                        {VX_GQ(q4_k_t2), VX_GQ(q4_k_t3)}};
+#undef VX_GQ
+#undef VX_GQ1
+    vx_gemv_args a{};
+    a.w = (const uint8_t*)w->base;
+    a.row_stride = w->row_stride_bytes;
+    a.xs_k = cx.l.stride[2];
+    a.xs_b = cx.l.stride[3];
+    a.ys_m = cy.l.stride[2];
+    a.ys_b = cy.l.stride[3];
+    a.M = w->rows;
+    a.K = w->cols;
+    a.nunits = w->cols / 64u;
+    a.x_vec = (a.xs_k == 1 && aligned16(cx.ptr) && a.xs_b % 4 == 0) ? 1u : 0u;
+    const int k = tab[q_index(w->qtype)][nt - 2][cfg][a.x_vec ? 0 : 1];
+    const uint32_t rows = kGemmQRows[cfg], cols = kGemmQCols[cfg];
+    const uint32_t nrow = (uint32_t)(((uint64_t)a.M + rows - 1u) / rows);
+    size_t lds;  // the waves' partial sums, or x (two buffers), W's rows of an item and the sums of x
+    if (cfg < 3) lds = (size_t)8u * rows * cols * 4u;
+    else lds = (size_t)2u * 8u * (uint32_t)nt * 1024u + rows * (w->qtype == VX_Q8_0 ? 272u : 144u) +
+               (w->qtype == VX_Q8_0 ? 0u : 2u * 8u * 2u * cols * 4u);
+    // a grid holds fewer than 2^32 threads: columns in slices of at most 2^22 workgroups
+    const uint32_t slice = std::max(1u, (1u << 22) / nrow);
+    for (uint64_t b0 = 0; b0 < B; b0 += (uint64_t)slice * cols) {
+        a.B = (uint32_t)std::min<uint64_t>(B - b0, (uint64_t)slice * cols);
+        a.x = (const float*)(cx.ptr + 4ull * b0 * (uint64_t)a.xs_b);
+        a.y = (float*)(cy.ptr + 4ull * b0 * (uint64_t)a.ys_b);
+        const int s = launch(ctx, k, dim3(nrow * ((a.B + cols - 1u) / cols)), dim3(512), lds, stream, a);
+        if (s) return s;
+    }
+    return VX_OK;
+}
+
 // Where the batched GEMV's activation split may go: nowhere (vx_gemv_q /
 // _ex), a caller's workspace (vx_gemv_q_ws) or the module scratch
 // (vx_gemv_q_noalloc).
@@ -880,6 +958,13 @@ static int run_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y, const vx_
                 std::to_string(nb) + " bytes of device memory: pass a workspace (vx_gemv_q_ws)";
             return fail(VX_ERR_UNSUPPORTED, m.c_str());
         }
+        if (q.base && B > 16u && gemm_q_ok(w)) {
+            // two bf16 terms of x are closer to it than the int8 split, and
+            // W streams once per tile of columns instead of once per 16
+            double us = 0.0;
+            const int cfg = gemm_q_choose(ctx, w->qtype, M, K, B, 2, &us);
+            if (us < gemv_xq_us(w->qtype, M, K, B)) return launch_gemm_q(ctx, stream, cy, w, cx, B, 2, cfg);
+        }
         if (q.base) {
             if ((s = launch_quantize_x(ctx, stream, &q, cx))) return s;
             return launch_gemv_xq(ctx, stream, cy, w, &q);
@@ -887,13 +972,22 @@ static int run_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y, const vx_
         // no memory for the split: exact f32 x (the VX_GEMV_X_F32 kernels)
         x_f32 = true;
     }
+    if (B > 4u && x_f32 && gemm_q_ok(w)) {
+        // exact x on the matrix cores, as three bf16 terms. Up to four columns
+        // the f32 vector kernels below are as fast or faster (1024 x 4096 B =
+        // 4 8.3 against 10.6 us, 16448 x 4096 37 against 30; B = 8 17.3 / 10.7
+        // and 78 / 31 us).
+        double us = 0.0;
+        const int cfg = gemm_q_choose(ctx, w->qtype, M, K, B, 3, &us);
+        return launch_gemm_q(ctx, stream, cy, w, cx, B, 3, cfg);
+    }
     // batch-1 kernel: the persistent one, or the per-row-group one when x
     // does not fit the persistent kernel's LDS (K > 16384); int8 x unless
     // VX_GEMV_X_F32
     uint32_t b0 = 0;
     while (b0 < B) {
         const uint32_t rem = B - b0;
-        const int NB = rem >= 16 ? 16 : rem >= 8 ? 8 : rem >= 4 ? 4 : rem >= 2 ? 2 : 1;
+        const int NB = rem >= 4 ? 4 : rem >= 2 ? 2 : 1;
         a.x = (const float*)(cx.ptr + 4ull * (uint64_t)b0 * (uint64_t)cx.l.stride[3]);
         a.y = (float*)(cy.ptr + 4ull * (uint64_t)b0 * (uint64_t)cy.l.stride[3]);
         a.B = NB;
@@ -961,7 +1055,7 @@ static int run_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y, const vx_
             rows_per_wg = 4u * R;
             lds = (size_t)NB * 16u * a.upitch * 16u;
         } else {
-            const uint32_t LPR = NB <= 4 ? 64u : NB == 8 ? 32u : 16u;
+            const uint32_t LPR = 64u;
             // Largest multiple of LPR whose [NB][16][pitch] float4 block fits.
             // An odd pitch keeps the staging stores conflict free; an even
             // one is used when the odd pitch would not fit.
