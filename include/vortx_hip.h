@@ -135,7 +135,12 @@ int vx_device_info(vx_ctx ctx, int* device, int* num_cus);
  * out is [.., M, N], lhs [.., M, K], rhs [.., K, N]. Arbitrary strides
  * (transposed views included). Kernel choice by shape: the naive kernel
  * when M < 32 and N < 32 (the reference's rule, :111-112), an f32 GEMV
- * when N == 1, otherwise the MFMA tiled kernel. out is only written. */
+ * when N == 1, otherwise the MFMA tiled kernels. out is only written.
+ * The tiled kernels give f32 results: except for a short K, operands are taken
+ * as the exact sums of three bf16 terms each and the six largest of the nine
+ * products of terms are added in f32 on the bf16 matrix cores (as close to the
+ * exact result as f32 products or closer); outputs that are not finite, or too
+ * small for the smaller terms, are formed from the f32 operands. */
 int vx_gemm_f32(vx_ctx ctx, vx_stream stream, const vx_mview* out,
                 const vx_cview* lhs, const vx_cview* rhs);
 
@@ -159,11 +164,11 @@ typedef enum vx_gemm_flags {
      * of TensorLayout::broadcast (src/shapes.rs:346-391) that the reference
      * leaves as a TODO in Gemm::dispatch (src/linalg/gemm.rs:64). */
     VX_GEMM_BROADCAST = 1,
-    /* Tile shape of the MFMA kernel, for callers that pin it (all give the
+    /* Tile shape of the MFMA kernels, for callers that pin it (all give the
      * same bits; by default the one that fills the GPU best is taken):
-     * 128 x 128, 128 x 256 or 64 x 64 output tiles. Exclusive; ignored on
-     * the naive and GEMV routes; WIDE and SMALL apply to operands whose A is
-     * contiguous along K and B along K or N (others keep 128 x 128). */
+     * 128 x 128, 256 x 128 (short K: 128 x 256) or 64 x 64 output tiles.
+     * Exclusive; ignored on the naive and GEMV routes and where few outputs
+     * are computed with K split over a workgroup instead. */
     VX_GEMM_TILE_NARROW = 2,
     VX_GEMM_TILE_WIDE = 4,
     VX_GEMM_TILE_SMALL = 8

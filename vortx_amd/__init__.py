@@ -200,7 +200,7 @@ class Gemm(_Context):
         """out = alpha * (lhs x rhs) + beta * out (vx_gemm_f32_ex); out is not
         read when beta == 0. ``broadcast``: batch dims of lhs / rhs of size 1
         are reused along out's (src/shapes.rs:346-391 semantics). ``tile``:
-        "narrow" / "wide" / "small" pins the MFMA kernel's 128 x 128 / 128 x 256 /
+        "narrow" / "wide" / "small" pins the MFMA kernels' 128 x 128 / 256 x 128 /
         64 x 64 output tiles (same bits every way), "auto" lets the library choose."""
         o, l, r = _view_of(out, True), _view_of(lhs, False), _view_of(rhs, False)
         flags = (_ffi.VX_GEMM_BROADCAST if broadcast else 0) | {"auto": 0, "narrow": _ffi.VX_GEMM_TILE_NARROW,

@@ -28,7 +28,8 @@ ARCH = "gfx950"
 
 # module symbol -> kernel source
 MODULES = {"vx_co_gemm": "gemm.hip", "vx_co_gemv_q": "gemv_q.hip", "vx_co_copy": "copy.hip",
-           "vx_co_quantize": "quantize.hip", "vx_co_gemm_q": "gemm_q.hip"}
+           "vx_co_quantize": "quantize.hip", "vx_co_gemm_q": "gemm_q.hip",
+           "vx_co_gemm_bf": "gemm_bf.hip"}
 HOST_SOURCES = ["vx_host.cpp", "vx_layout.cpp", "vx_gguf.cpp"]
 
 HIPCC_FLAGS = [

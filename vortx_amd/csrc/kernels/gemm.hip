@@ -5,7 +5,8 @@
 //                  rounding per multiply and per add: the summation order of
 //                  the reference's gemm_naive / gemm_tiled
 //                  (vortx-shaders/src/linalg/gemm.rs:84-171, 225-235).
-//  vx_gemm_mfma_*  128x128 output tile per workgroup (4 wave64 in 2x2, each
+//  vx_gemm_mfma_*  short K and not many outputs, contiguous aligned rows (the
+//                  rest: gemm_bf.hip): 128x128 output tile per workgroup (4 wave64 in 2x2, each
 //                  64x64 = 2x2 v_mfma_f32_32x32x2f32 accumulators), K staged
 //                  16 at a time through double-buffered LDS (k-major, one
 //                  barrier per stage). Operand loads are 128-bit along the
@@ -33,7 +34,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // Operand access modes (chosen on the host from strides and alignment).
 #define MODE_KC 0  // contiguous along K, rows 16-byte aligned
 #define MODE_XC 1  // contiguous along M (for A) / N (for B), 16-byte aligned
-#define MODE_GEN 2 // anything else: scalar loads
 
 // Output epilogue: alpha * acc + beta * c, where c is read only when
 // beta != 0 (the BLAS convention: out may hold NaN when beta == 0). With
@@ -95,7 +95,7 @@ __device__ __forceinline__ void vx_load_frag(vx_frag<MODE, TX>& f, const float* 
                 for (int e = 0; e < 4; ++e) f.v[4 * i + e] = (x < X && k + e < K) ? p[e] : 0.f;
             }
         }
-    } else if constexpr (MODE == MODE_XC) {
+    } else {
         // 16 k-rows of TX / 4 float4 along x: element (k = f / QX, x = 4(f % QX)).
 #pragma unroll
         for (int i = 0; i < TX / 64; ++i) {
@@ -109,14 +109,6 @@ __device__ __forceinline__ void vx_load_frag(vx_frag<MODE, TX>& f, const float* 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) f.v[4 * i + e] = (k < K && x + e < X) ? p[e] : 0.f;
             }
-        }
-    } else {
-        // scalar: element (k = f / TX, x = f % TX), f = t + 256 i.
-#pragma unroll
-        for (int i = 0; i < TX / 16; ++i) {
-            const uint32_t fi = t + 256u * i;
-            const uint32_t k = k0 + fi / TX, x = x0 + fi % TX;
-            f.v[i] = (k < K && x < X) ? base[(int64_t)k * sk + (int64_t)x * sx] : 0.f;
         }
     }
 }
@@ -136,7 +128,7 @@ __device__ __forceinline__ void vx_load_frag_full(vx_frag<MODE, TX>& f, const fl
             const f32x4 q = *(const f32x4*)(base + (int64_t)(x0 + (fi >> 2)) * sx + k0 + 4u * (fi & 3u));
             f.v[4 * i + 0] = q.x; f.v[4 * i + 1] = q.y; f.v[4 * i + 2] = q.z; f.v[4 * i + 3] = q.w;
         }
-    } else if constexpr (MODE == MODE_XC) {
+    } else {
         // the stage's offset k0 * sk is uniform (scalar); the per-thread part
         // is the same every stage, so the compiler keeps it out of the loop
         // (written as one product, it cost a 64-bit multiply per load and stage)
@@ -146,12 +138,6 @@ __device__ __forceinline__ void vx_load_frag_full(vx_frag<MODE, TX>& f, const fl
             const uint32_t fi = t + 256u * i;
             const f32x4 q = *(const f32x4*)(stage + ((int64_t)(fi / QX) * sk + x0 + 4u * (fi % QX)));
             f.v[4 * i + 0] = q.x; f.v[4 * i + 1] = q.y; f.v[4 * i + 2] = q.z; f.v[4 * i + 3] = q.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < TX / 16; ++i) {
-            const uint32_t fi = t + 256u * i;
-            f.v[i] = base[(int64_t)(k0 + fi / TX) * sk + (int64_t)(x0 + fi % TX) * sx];
         }
     }
 }
@@ -169,18 +155,12 @@ __device__ __forceinline__ void vx_store_frag(const vx_frag<MODE, TX>& f, float*
 #pragma unroll
             for (int e = 0; e < 4; ++e) S[(k + e) * LD + x] = f.v[4 * i + e];
         }
-    } else if constexpr (MODE == MODE_XC) {
+    } else {
 #pragma unroll
         for (int i = 0; i < TX / 64; ++i) {
             const uint32_t fi = t + 256u * i;
             const uint32_t k = fi / QX, x = 4u * (fi % QX);
             *(f32x4*)(S + k * LD + x) = f32x4{f.v[4 * i], f.v[4 * i + 1], f.v[4 * i + 2], f.v[4 * i + 3]};
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < TX / 16; ++i) {
-            const uint32_t fi = t + 256u * i;
-            S[(fi / TX) * LD + fi % TX] = f.v[i];
         }
     }
 }
@@ -368,10 +348,9 @@ __device__ __forceinline__ void vx_gemm_mfma(const vx_gemm_args& p) {
 // 256-thread workgroups per CU (the wide kernels use ~245 under WPE 2: two). The two-stage prefetch's second register
 // buffer needs ~150-166 registers; squeezed into WPE 4's 128 (four
 // workgroups per CU) it ran slower: 4096^3 118.7 vs 123.5 TFLOP/s, B
-// transposed 126.4 vs 134.9, 1024^3 25.5 vs 29.8 (same-box A/B). The
-// all-scalar mode needs more and is left uncapped (WPE 1).
-#define VX_GEMM_MFMA(AM, BM, NAME, WPE)                                                              \
-    extern "C" __global__ __launch_bounds__(VX_WG) __attribute__((amdgpu_waves_per_eu(WPE, 4)))    \
+// transposed 126.4 vs 134.9, 1024^3 25.5 vs 29.8 (same-box A/B).
+#define VX_GEMM_MFMA(AM, BM, NAME)                                                                   \
+    extern "C" __global__ __launch_bounds__(VX_WG) __attribute__((amdgpu_waves_per_eu(3, 4)))      \
     void vx_gemm_mfma_##NAME(vx_gemm_args p) {                                                       \
         vx_gemm_mfma<AM, BM, 128, 128>(p);                                                              \
     }
@@ -388,14 +367,9 @@ __device__ __forceinline__ void vx_gemm_mfma(const vx_gemm_args& p) {
         vx_gemm_mfma<AM, BM, 64, 64>(p);                                                             \
     }
 // Suffix letters: A mode then B mode; k = contiguous along K,
-// x = contiguous along M / N, g = generic.
-VX_GEMM_MFMA(MODE_KC, MODE_XC, kx, 3)  // row-major A, row-major B
-VX_GEMM_MFMA(MODE_KC, MODE_KC, kk, 3)  // row-major A, B = transposed view of [N, K]
-VX_GEMM_MFMA(MODE_XC, MODE_XC, xx, 3)
-VX_GEMM_MFMA(MODE_XC, MODE_KC, xk, 3)
-VX_GEMM_MFMA(MODE_GEN, MODE_GEN, gg, 1)
-VX_GEMM_MFMA(MODE_KC, MODE_GEN, kg, 3)
-VX_GEMM_MFMA(MODE_GEN, MODE_XC, gx, 3)
+// x = contiguous along M / N.
+VX_GEMM_MFMA(MODE_KC, MODE_XC, kx)  // row-major A, row-major B
+VX_GEMM_MFMA(MODE_KC, MODE_KC, kk)  // row-major A, B = transposed view of [N, K]
 VX_GEMM_MFMA_W(MODE_KC, MODE_XC, kx)
 VX_GEMM_MFMA_W(MODE_KC, MODE_KC, kk)
 VX_GEMM_MFMA_S(MODE_KC, MODE_XC, kx)

@@ -1,0 +1,534 @@
+// gemm_bf.hip — f32 GEMM on the bf16 matrix cores, on canonical [n, c, rows,
+// cols] views (any strides; batch dims folded into grid z).
+//
+// Each operand element is the exact sum of three bf16 terms (vx_bf16.hpp), and
+// six of the nine products of terms are formed, down to 2^-16 of the largest;
+// the others are below 2^-24 of a product, the size of one f32 rounding.
+// Products of bf16 values are exact in f32 and the matrix cores add them in
+// f32, so the result is as close to the exact one as that of f32 MFMAs (closer:
+// at K = 4096 7.1e-7 off 64 bits against 1.15e-6, with fewer additions in
+// f32), at six times the MFMA work but sixteen times the rate.
+//
+// Measured (graph-replayed, same box, against the f32 MFMA kernels): 4096^3 980
+// -> 650 us (212 TFLOP/s of f32 work, 1270 of bf16; a bf16 product of that size
+// by the vendor's library 1370 on this card), 4096 x 11008 x 4096 2720 -> 1870,
+// 1024^3 26 -> 23.5, 1000 x 1111 x 777 with odd strides 119 -> 28, 8 x 11008 x
+// 4096 154 -> 53 (K split), 64 x 64 x 4096 394 -> 25.5 (K split). The large
+// shapes are bound by the matrix cores and the card's power, the smaller ones
+// by the stages' serial steps (load, convert, store, barrier, read, multiply)
+// with one workgroup per CU.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "../vx_kargs.h"
+#include "vx_bf16.hpp"
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Operand access: "x" is the non-K dimension (M for A, N for B).
+#define MODE_K 0  // stride 1 along K
+#define MODE_X 1  // any strides; best with stride 1 along x
+
+__device__ __forceinline__ void vx_epilogue(float* c, float acc, float alpha, float beta) {
+    *c = beta == 0.f ? alpha * acc : alpha * acc + beta * *c;
+}
+
+// Loads of one operand's BK x T slab of a stage: pieces of 8 k-elements of one
+// x, P per thread. MODE_K: BK / 8 consecutive lanes cover a row's BK elements
+// (two 16-byte loads each, 4-byte aligned); else consecutive lanes are
+// consecutive in x (eight 4-byte loads, one row of k each). x past the operand
+// repeats its last one (those outputs are not written). NTH threads share the
+// slab (the workgroup, or half of it: the others then do the same ones).
+template <int MODE, int T, int BK, int NTH, int D>
+struct vx_slab {
+    static constexpr int KG = BK / 8, P = T * KG / NTH;
+    static_assert(P * NTH == T * KG, "whole pieces");
+    float r[D][P][8];  // D stages in flight
+    const float* p[P];
+    float mx[P];  // largest |element| seen
+
+    static __device__ __forceinline__ uint32_t px(int u) {
+        const uint32_t i = threadIdx.x % NTH + (uint32_t)(NTH * u);
+        return MODE == MODE_K ? i / KG : i % T;
+    }
+    static __device__ __forceinline__ uint32_t pk(int u) {
+        const uint32_t i = threadIdx.x % NTH + (uint32_t)(NTH * u);
+        return MODE == MODE_K ? i % KG : __builtin_amdgcn_readfirstlane(i / T);  // T is a multiple of 64
+    }
+    __device__ __forceinline__ void init(const float* base, int64_t sx, uint32_t x0, uint32_t X) {
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const uint32_t x = min(x0 + px(u), X - 1u);
+            p[u] = MODE == MODE_K ? base + (int64_t)x * sx + 8u * pk(u) : base + (int64_t)x * sx;
+            mx[u] = 0.f;
+        }
+    }
+    // a stage inside K
+    __device__ __forceinline__ void load(int d, int u, int64_t sk, uint32_t k0) {
+        if constexpr (MODE == MODE_K) {
+            const f32x4_a4 a = *(const f32x4_a4*)(p[u] + k0), b = *(const f32x4_a4*)(p[u] + k0 + 4);
+            r[d][u][0] = a.x; r[d][u][1] = a.y; r[d][u][2] = a.z; r[d][u][3] = a.w;
+            r[d][u][4] = b.x; r[d][u][5] = b.y; r[d][u][6] = b.z; r[d][u][7] = b.w;
+        } else {
+            const int64_t k = (int64_t)(k0 + 8u * pk(u)) * sk;  // uniform over the wave
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r[d][u][j] = p[u][k + j * sk];
+        }
+    }
+    // the last stage, zeros past K
+    __device__ __forceinline__ void load_tail(int d, int u, int64_t sk, uint32_t k0, uint32_t K) {
+        const uint32_t kp = k0 + 8u * pk(u);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            // (loads from clamped addresses, so that all are in flight at once)
+            const uint32_t k = min(kp + (uint32_t)j, K - 1u);
+            const float e = MODE == MODE_K ? (p[u] - 8u * pk(u))[k] : p[u][(int64_t)k * sk];
+            r[d][u][j] = kp + (uint32_t)j < K ? e : 0.f;
+        }
+    }
+    // terms of piece u to LDS: [k16][x / 32][term][64 lanes], lane (n, g) of
+    // an MFMA operand (row n, k 8g..8g+7) at g 32 + (n ^ 4 kg), kg = 2 k16 + g:
+    // the xor spreads the pieces that 8 consecutive lanes store over the banks
+    __device__ __forceinline__ void store(int d, int u, u32x4* S) {
+        u32x4 t[3];
+        vx_split8_rne(r[d][u], t);
+#pragma unroll
+        for (int j = 0; j < 8; j += 2)
+            mx[u] = fmaxf(fmaxf(__builtin_fabsf(r[d][u][j]), __builtin_fabsf(r[d][u][j + 1])), mx[u]);
+        const uint32_t x = px(u), kg = pk(u);
+        u32x4* o = S + (((kg >> 1) * (T / 32) + (x >> 5)) * 3u) * 64u + (kg & 1u) * 32u + ((x & 31u) ^ (4u * kg));
+#pragma unroll
+        for (int k = 0; k < 3; ++k) o[64 * k] = t[k];
+    }
+};
+
+// Element (row, col) the plain way: an output that is not finite (the terms of
+// an infinity hold a NaN), or whose row of A or column of B holds nothing
+// above 2^-109 (its third terms fall below bf16's subnormals), or whose
+// products fall below 2^-80 (so would some of their parts).
+__device__ __forceinline__ float vx_gemm_bf_redo(const vx_gemm_args& p, const float* a, const float* b) {
+    float s = 0.f;
+    for (uint32_t k = 0; k < p.K; ++k) s = __builtin_fmaf(a[(int64_t)k * p.as[3]], b[(int64_t)k * p.bs[2]], s);
+    return s;
+}
+
+extern __shared__ __align__(16) uint8_t vx_bf_lds[];
+
+// A stage is 32 ST elements of K. Even and odd steps of 16 are added up apart and
+// the two sums at the end, in every tile shape, so that all
+// give the same bits: a wave holds both (HS 1), or, where tiles are few or
+// small, twice as many waves hold one each (HS 2) and meet in LDS.
+template <int AM, int BM, int TM, int TN, int WM, int WN, int HS, int ST>
+__device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
+    constexpr int BK = 32 * ST, KH = 2 * ST, NTH = 64 * WM * WN * HS, MI = TM / WM / 32, NJ = TN / WN / 32, NA = 2 / HS;
+    constexpr int D = HS;  // stages requested ahead of the one being converted (registers allow two with HS 2)
+    constexpr uint32_t SA = KH * (TM / 32) * 3u * 64u, SB = KH * (TN / 32) * 3u * 64u;  // pieces per buffer
+    u32x4* SAp = (u32x4*)vx_bf_lds;
+    u32x4* SBp = SAp + 2u * SA;
+
+    // Tile order: workgroup ids are regrouped per XCD (dealt round robin over
+    // 8), then walked in groups of 8 tile rows, so that an XCD's resident
+    // tiles share panels of A and B in its L2.
+    const uint32_t nt = p.tiles_m * p.tiles_n;
+    uint32_t bid = blockIdx.x;
+    if ((nt & 7u) == 0) bid = (bid & 7u) * (nt >> 3) + (bid >> 3);
+    const uint32_t group = 8u * p.tiles_n;
+    const uint32_t first_m = (bid / group) * 8u;
+    const uint32_t gsize = min(p.tiles_m - first_m, 8u);
+    const uint32_t m0 = (first_m + (bid % group) % gsize) * TM, n0 = (bid % group) / gsize * TN;
+    const uint32_t z = blockIdx.z;
+    const uint32_t bn = z / p.batch_c, bc = z % p.batch_c;
+    const float* A = p.a + bn * p.as[0] + bc * p.as[1];
+    const float* B = p.b + bn * p.bs[0] + bc * p.bs[1];
+    float* C = p.c + bn * p.cs[0] + bc * p.cs[1];
+
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wh = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN, n = lane & 31u, g = lane >> 5;
+
+    f32x16 acc[NA][MI][NJ];
+#pragma unroll
+    for (int q = 0; q < NA; ++q)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[q][i][j][v] = 0.f;
+
+    // DUTY: small tiles have a piece for every thread in A and B together; the
+    // first half of the waves takes A's, the second half B's
+    constexpr bool DUTY = (TM + TN) * (BK / 8) == NTH;
+    vx_slab<AM, TM, BK, DUTY ? NTH / 2 : NTH, D> a;
+    vx_slab<BM, TN, BK, DUTY ? NTH / 2 : NTH, D> b;
+    constexpr int PA = a.P, PB = b.P;
+    const bool dutyb = DUTY && wave >= (uint32_t)(NTH / 128);
+    a.init(A, p.as[2], m0, p.M);
+    b.init(B, p.bs[3], n0, p.N);
+
+    const uint32_t nkf = p.K / BK;
+    // accumulator q: half h of the stage in buffer buf
+    auto mult = [&](uint32_t buf, int q, uint32_t h) {
+        const uint32_t slot = g * 32u + (n ^ (4u * (2u * h + g)));
+        const u32x4* sa = SAp + buf * SA + (h * (TM / 32) + wm * MI) * 192u + slot;
+        const u32x4* sb = SBp + buf * SB + (h * (TN / 32) + wn * NJ) * 192u + slot;
+        bf16x8 fa[MI][3], fb[NJ][3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) fa[i][k] = __builtin_bit_cast(bf16x8, sa[i * 192 + k * 64]);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) fb[j][k] = __builtin_bit_cast(bf16x8, sb[j * 192 + k * 64]);
+        }
+        constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};  // smallest products first
+#pragma unroll
+        for (int e = 0; e < 6; ++e)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    acc[q][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][TA[e]], fb[j][TB[e]], acc[q][i][j], 0, 0, 0);
+    };
+    // stage st's elements to registers (slot d), and from there to LDS
+    auto load = [&](int d, uint32_t st) {
+        const uint32_t k0 = min(st, nkf - 1u) * BK;
+        if (!DUTY || !dutyb) {
+#pragma unroll
+            for (int u = 0; u < PA; ++u) a.load(d, u, p.as[3], k0);
+        }
+        if (!DUTY || dutyb) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u) b.load(d, u, p.bs[2], k0);
+        }
+    };
+    auto store = [&](int d, uint32_t buf) {
+        if (!DUTY || !dutyb) {
+#pragma unroll
+            for (int u = 0; u < PA; ++u) a.store(d, u, SAp + buf * SA);
+        }
+        if (!DUTY || dutyb) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u) b.store(d, u, SBp + buf * SB);
+        }
+    };
+    // stage st from its buffer; stage st + 1 is converted to the other one
+    // from slot d, which then takes stage st + 1 + D (clamped to the last)
+    auto stage = [&](uint32_t st, int d) __attribute__((always_inline)) {
+        const uint32_t buf = st & 1u, k2 = min(st + 1u + (uint32_t)D, nkf - 1u) * BK;
+#pragma unroll
+        for (int q = 0; q < NA * ST; ++q) {
+            __builtin_amdgcn_sched_barrier(0);
+            mult(buf, q % NA, HS == 1 ? (uint32_t)q : 2u * (uint32_t)q + wh);
+            if constexpr (!DUTY) {
+#pragma unroll
+                for (int u = 0; u < PA + PB; ++u) {
+                    if (u * (NA * ST) / (PA + PB) != q) continue;
+                    if (u < PA) {
+                        a.store(d, u, SAp + (buf ^ 1u) * SA);
+                        a.load(d, u, p.as[3], k2);
+                    } else {
+                        b.store(d, u - PA, SBp + (buf ^ 1u) * SB);
+                        b.load(d, u - PA, p.bs[2], k2);
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < 6 * MI * NJ; ++m) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, MI * NJ == 1 ? 10 : 4, 0);
+                }
+            }
+        }
+        if constexpr (DUTY) {
+            store(d, buf ^ 1u);
+            load(d, st + 1u + (uint32_t)D);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+    if (nkf) {
+        load(0, 0u);
+        if (D == 2) load(1, 1u);
+        store(0, 0u);
+        load(0, (uint32_t)D);
+        __syncthreads();
+        uint32_t st = 0;
+        if constexpr (D == 1) {
+            for (; st < nkf; ++st) stage(st, 0);
+        } else {
+            for (; st + 2u <= nkf; st += 2u) {
+                stage(st, 1);
+                stage(st + 1u, 0);
+            }
+            if (st < nkf) stage(st, 1);
+        }
+    }
+    if (p.K % BK) {
+        // (the buffers' last readers finished before a barrier)
+        if (!DUTY || !dutyb) {
+#pragma unroll
+            for (int u = 0; u < PA; ++u) a.load_tail(0, u, p.as[3], nkf * BK, p.K);
+        }
+        if (!DUTY || dutyb) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u) b.load_tail(0, u, p.bs[2], nkf * BK, p.K);
+        }
+        store(0, 0u);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NA * ST; ++q) mult(0u, q % NA, HS == 1 ? (uint32_t)q : 2u * (uint32_t)q + wh);
+        __syncthreads();
+    }
+    // Even + odd, to acc[0] (HS 2: of the even waves). Beside it one word says
+    // whether a thread saw only small elements in a piece (8 elements of a row
+    // or column per stage) with any: some output may then need a closer look.
+    uint32_t* word = (uint32_t*)(SBp + 2u * SB);
+    bool small = false;
+#pragma unroll
+    for (int u = 0; u < PA; ++u) small |= a.mx[u] < 0x1p-40f && a.mx[u] > 0.f;
+#pragma unroll
+    for (int u = 0; u < PB; ++u) small |= b.mx[u] < 0x1p-40f && b.mx[u] > 0.f;
+    if (threadIdx.x == 0u) *word = 0u;
+    float* red = (float*)vx_bf_lds + wave % (WM * WN) * (MI * NJ * 1024u) + lane;
+    if (HS == 2 && wh) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) red[((i * NJ + j) * 16 + v) * 64] = acc[0][i][j][v];
+    }
+    __syncthreads();
+    if (small) *word = 1u;
+    if (!wh) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                if constexpr (HS == 1) acc[0][i][j] += acc[1][i][j];
+                else {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[0][i][j][v] += red[((i * NJ + j) * 16 + v) * 64];
+                }
+            }
+    }
+    __syncthreads();
+    const bool look = *word != 0u;
+    const uint32_t rt0 = wm * (32u * MI) + 4u * g, ct0 = wn * (32u * NJ) + n;
+    float* c0 = C + (int64_t)(m0 + rt0) * p.cs[2] + (int64_t)(n0 + ct0) * p.cs[3];
+    uint64_t again = 0;  // outputs to form the plain way
+    static_assert(MI * NJ * 16 <= 64, "one bit per output of a lane");
+    if (!wh) {
+        float f = 0.f;  // NaN when an output is not finite
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) f = __builtin_fmaf(acc[0][i][j][v], 0.f, f);
+        if (!__any(f != 0.f || look) && m0 + TM <= p.M && n0 + TN <= p.N) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        vx_epilogue(c0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * p.cs[2] + (int64_t)(32 * j) * p.cs[3],
+                                    acc[0][i][j][v], p.alpha, p.beta);
+            return;  // (look is clear: no barrier follows for the workgroup)
+        }
+    }
+    uint32_t* mx = (uint32_t*)vx_bf_lds;  // [TM + TN] the largest |element| of each row of A and column of B
+    if (look) {
+        for (uint32_t i = threadIdx.x; i < TM + TN; i += NTH) mx[i] = 0u;
+        __syncthreads();
+        if (!DUTY || !dutyb) {
+#pragma unroll
+            for (int u = 0; u < PA; ++u) atomicMax(&mx[a.px(u)], __float_as_uint(a.mx[u]));
+        }
+        if (!DUTY || dutyb) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u) atomicMax(&mx[TM + b.px(u)], __float_as_uint(b.mx[u]));
+        }
+        __syncthreads();
+    }
+    if (wh) return;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const uint32_t ct = ct0 + 32u * j;
+        const float cm = look ? __uint_as_float(mx[TM + ct]) : 1.f;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const uint32_t rt = rt0 + 32u * i + 8u * (v >> 2) + (v & 3);
+                const float rm = look ? __uint_as_float(mx[rt]) : 1.f;
+                if (m0 + rt < p.M && n0 + ct < p.N) {
+                    const bool tiny = (rm * cm < 0x1p-80f || fminf(rm, cm) < 0x1p-109f) && rm > 0.f && cm > 0.f;
+                    if (__builtin_fabsf(acc[0][i][j][v]) < __builtin_inff() && !tiny)
+                        vx_epilogue(c0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * p.cs[2] + (int64_t)(32 * j) * p.cs[3],
+                                    acc[0][i][j][v], p.alpha, p.beta);
+                    else
+                        again |= 1ull << ((j * MI + i) * 16 + v);
+                }
+            }
+    }
+    while (again) {
+        const uint32_t o = (uint32_t)__builtin_ctzll(again), v = o & 15u, i = (o >> 4) % MI, j = (o >> 4) / MI;
+        again &= again - 1u;
+        const uint32_t row = m0 + rt0 + 32u * i + 8u * (v >> 2) + (v & 3u), col = n0 + ct0 + 32u * j;
+        const float s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
+        vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+    }
+}
+
+// 32 x 32 tiles with K split over the 8 waves of a workgroup: for shapes with
+// too few outputs to fill the GPU otherwise (a few rows through a wide layer, a
+// small output from a long K). Wave w takes the 32-element chunks w, w + 8, ...
+// of K straight from memory to registers (no LDS, no barrier in the loop, one
+// chunk ahead), and the waves' sums meet in LDS in wave order.
+template <int MODE>
+struct vx_chunk {  // one operand's 32 k of lane (n, g)'s x: k16 step h, elements 8g..8g+7
+    float r[2][8];
+    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0, uint32_t g) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t k = k0 + 16u * h + 8u * g;
+            if constexpr (MODE == MODE_K) {
+                const f32x4_a4 a = *(const f32x4_a4*)(p + k), b = *(const f32x4_a4*)(p + k + 4);
+                r[h][0] = a.x; r[h][1] = a.y; r[h][2] = a.z; r[h][3] = a.w;
+                r[h][4] = b.x; r[h][5] = b.y; r[h][6] = b.z; r[h][7] = b.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) r[h][j] = p[(int64_t)(k + (uint32_t)j) * sk];
+            }
+        }
+    }
+    __device__ __forceinline__ void load_tail(const float* p, int64_t sk, uint32_t k0, uint32_t g, uint32_t K) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t k = k0 + 16u * h + 8u * g + (uint32_t)j, kc = min(k, K - 1u);
+                const float e = p[MODE == MODE_K ? (int64_t)kc : (int64_t)kc * sk];  // (clamped: no branches between the loads)
+                r[h][j] = k < K ? e : 0.f;
+            }
+    }
+};
+
+template <int AM, int BM>
+__device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
+    constexpr uint32_t NWV = 8;
+    const uint32_t t = threadIdx.x, lane = t & 63u, n = lane & 31u, g = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t nt = p.tiles_m * p.tiles_n;
+    uint32_t bid = blockIdx.x;  // tiles that share columns of B follow each other on one XCD
+    if ((nt & 7u) == 0) bid = (bid & 7u) * (nt >> 3) + (bid >> 3);
+    const uint32_t m0 = bid % p.tiles_m * 32u, n0 = bid / p.tiles_m * 32u;
+    const uint32_t z = blockIdx.z;
+    const uint32_t bn = z / p.batch_c, bc = z % p.batch_c;
+    const float* A = p.a + bn * p.as[0] + bc * p.as[1];
+    const float* B = p.b + bn * p.bs[0] + bc * p.bs[1];
+    float* C = p.c + bn * p.cs[0] + bc * p.cs[1];
+    const float* pa = A + (int64_t)min(m0 + n, p.M - 1u) * p.as[2];
+    const float* pb = B + (int64_t)min(n0 + n, p.N - 1u) * p.bs[3];
+
+    f32x16 acc[2];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.f;
+    float ma = 0.f, mb = 0.f;  // the largest |element| seen
+    auto mult = [&](const vx_chunk<AM>& a, const vx_chunk<BM>& b) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            u32x4 ta[3], tb[3];
+            vx_split8_rne(a.r[h], ta);
+            vx_split8_rne(b.r[h], tb);
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                ma = fmaxf(fmaxf(__builtin_fabsf(a.r[h][j]), __builtin_fabsf(a.r[h][j + 1])), ma);
+                mb = fmaxf(fmaxf(__builtin_fabsf(b.r[h][j]), __builtin_fabsf(b.r[h][j + 1])), mb);
+            }
+            constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};  // smallest products first
+#pragma unroll
+            for (int e = 0; e < 6; ++e)
+                acc[h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ta[TA[e]]),
+                                                                 __builtin_bit_cast(bf16x8, tb[TB[e]]), acc[h], 0, 0, 0);
+        }
+    };
+    const uint32_t nck = p.K / 32u;  // whole chunks
+    if (wave < nck) {
+        vx_chunk<AM> a[2];
+        vx_chunk<BM> b[2];
+        const uint32_t last = (nck - 1u - wave) / NWV * NWV + wave;  // this wave's last chunk
+        auto load = [&](int d, uint32_t c) {
+            a[d].load(pa, p.as[3], min(c, last) * 32u, g);
+            b[d].load(pb, p.bs[2], min(c, last) * 32u, g);
+        };
+        load(0, wave);
+        load(1, wave + NWV);
+        uint32_t c = wave;
+        for (; c + NWV <= last; c += 2u * NWV) {
+            // (each chunk's next loads go out as soon as it is split: left free,
+            // the compiler issued both chunks' at the end of the round)
+            __builtin_amdgcn_sched_barrier(0);
+            mult(a[0], b[0]);
+            load(0, c + 2u * NWV);
+            __builtin_amdgcn_sched_barrier(0);
+            mult(a[1], b[1]);
+            load(1, c + 3u * NWV);
+        }
+        if (c <= last) mult(a[0], b[0]);
+    }
+    if (p.K % 32u != 0u && wave == nck % NWV) {
+        vx_chunk<AM> a;
+        vx_chunk<BM> b;
+        a.load_tail(pa, p.as[3], nck * 32u, g, p.K);
+        b.load_tail(pb, p.bs[2], nck * 32u, g, p.K);
+        mult(a, b);
+    }
+    // red[wave][v][lane], and the largest elements of the tile's rows of A and columns of B
+    float* red = (float*)vx_bf_lds;
+    uint32_t* mx = (uint32_t*)(red + NWV * 1024u);
+    if (t < 64u) mx[t] = 0u;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) red[wave * 1024u + (uint32_t)v * 64u + lane] = acc[0][v] + acc[1][v];
+    __syncthreads();
+    atomicMax(&mx[n], __float_as_uint(ma));
+    atomicMax(&mx[32u + n], __float_as_uint(mb));
+    __syncthreads();
+#pragma unroll
+    for (uint32_t o = t; o < 1024u; o += 64u * NWV) {
+        float s = red[o];
+#pragma unroll
+        for (uint32_t w = 1; w < NWV; ++w) s += red[w * 1024u + o];
+        const uint32_t l = o & 63u, v = o >> 6, rt = 8u * (v >> 2) + 4u * (l >> 5) + (v & 3u), ct = l & 31u;
+        const uint32_t row = m0 + rt, col = n0 + ct;
+        if (row >= p.M || col >= p.N) continue;
+        const float rm = __uint_as_float(mx[rt]), cm = __uint_as_float(mx[32u + ct]);
+        const bool tiny = (rm * cm < 0x1p-80f || fminf(rm, cm) < 0x1p-109f) && rm > 0.f && cm > 0.f;
+        if (!(__builtin_fabsf(s) < __builtin_inff()) || tiny)
+            s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
+        vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+    }
+}
+
+// 256 x 128 tiles (8 waves of 64 x 64), 128 x 128 (2 x 4 waves of 64 x 64) and
+// 64 x 64 (2 x 4 waves of 32 x 32): _s up to three workgroups per CU, _s2 one,
+// with half the barriers.
+#define VX_GEMM_BF1(AM, BM, NAME, WPE, ...)                                                              \
+    extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, WPE)))            \
+    void vx_gemm_bf_##NAME(vx_gemm_args p) {                                                             \
+        vx_gemm_bf<AM, BM, __VA_ARGS__>(p);                                                              \
+    }
+#define VX_GEMM_BF(AM, BM, NAME)                            \
+    VX_GEMM_BF1(AM, BM, NAME##_w, 2, 256, 128, 4, 2, 1, 1)  \
+    VX_GEMM_BF1(AM, BM, NAME##_n, 2, 128, 128, 2, 2, 2, 1)  \
+    VX_GEMM_BF1(AM, BM, NAME##_s2, 4, 64, 64, 2, 2, 2, 2)   \
+    VX_GEMM_BF1(AM, BM, NAME##_s, 6, 64, 64, 2, 2, 2, 1)    \
+    extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 3)))              \
+    void vx_gemm_bf_##NAME##_ks(vx_gemm_args p) {                                                        \
+        vx_gemm_bf_ks<AM, BM>(p);                                                                        \
+    }
+VX_GEMM_BF(MODE_K, MODE_X, kx)
+VX_GEMM_BF(MODE_K, MODE_K, kk)
+VX_GEMM_BF(MODE_X, MODE_X, xx)
+VX_GEMM_BF(MODE_X, MODE_K, xk)

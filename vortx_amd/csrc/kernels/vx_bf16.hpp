@@ -53,3 +53,23 @@ __device__ __forceinline__ void vx_split8(const float (&v)[8], u32x4 (&t)[NT]) {
         t[NT - 1][i] = NT == 3 ? vx_pk_hi(__float_as_uint(r[2 * i]), __float_as_uint(r[2 * i + 1]))
                                : vx_pk_bf16(r[2 * i], r[2 * i + 1]);
 }
+
+// v[0..8) as three terms of packed bf16 rounded to nearest, largest first:
+// exact down to bf16's smallest subnormal, and with |second| <= 2^-8 |v| and
+// |third| <= 2^-16 |v| of either sign, so that in a product of two such sums
+// the three smallest of the nine terms are below 2^-24 of it and average out.
+// |v| above 3.39e38 rounds to an infinity.
+__device__ __forceinline__ void vx_split8_rne(const float (&v)[8], u32x4 (&t)[3]) {
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = v[i];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t h = vx_pk_bf16(r[2 * i], r[2 * i + 1]);
+            t[k][i] = h;
+            r[2 * i] -= __uint_as_float(h << 16);
+            r[2 * i + 1] -= __uint_as_float(h & 0xFFFF0000u);
+        }
+}

@@ -33,6 +33,8 @@ extern const unsigned char vx_co_quantize[];
 extern const unsigned char vx_co_quantize_end[];
 extern const unsigned char vx_co_gemm_q[];
 extern const unsigned char vx_co_gemm_q_end[];
+extern const unsigned char vx_co_gemm_bf[];
+extern const unsigned char vx_co_gemm_bf_end[];
 }
 
 namespace vx {
@@ -71,8 +73,8 @@ static const char* const kKernelNames[K_COUNT] = {
 #undef K
 };
 // The embedded code objects; every kernel name is unique across them.
-static const unsigned char* const kModules[] = {vx_co_gemm, vx_co_gemv_q, vx_co_copy, vx_co_quantize, vx_co_gemm_q};
-constexpr int kNumModules = 5;
+static const unsigned char* const kModules[] = {vx_co_gemm, vx_co_gemv_q, vx_co_copy, vx_co_quantize, vx_co_gemm_q, vx_co_gemm_bf};
+constexpr int kNumModules = 6;
 constexpr int kModGemv = 1;  // the module holding vx_scratch
 
 }  // namespace vx
@@ -324,6 +326,64 @@ static int operand_mode(const Canon& c, int kdim, int xdim, uint32_t nb, uint32_
     return 2;
 }
 
+// The bf16 matrix-core GEMM (gemm_bf.hip): tile shapes and the K split.
+enum BfCfg { BF_W = 0, BF_N = 1, BF_S2 = 2, BF_S = 3, BF_KS = 4 };
+static const uint32_t kBfRows[5] = {256, 128, 64, 64, 32}, kBfCols[5] = {128, 128, 64, 64, 32};
+// Choice by estimated time in us, rounds of resident workgroups times what a
+// round costs: a fixed part (first loads, last stores) and one per 32 elements
+// of K. Measured (graph-replayed): 256 x 128 tiles 8 + 2.55 (4096^3 2 rounds
+// 650 us, 1024 x 1024 x 128, batch 32 4 rounds 74 us), 128 x 128 5.4 + 1.34
+// (2048^3 one round 91 us, 4096^3 four 690 us), 64 x 64 with long stages 2.8 +
+// 0.6 (1024^3 one round 23.5 us), with short ones, three per CU, per tile of a
+// CU 1 + 0.45 (1000 x 1111 x 777 31 us, against 42 with long stages); the K
+// split 2 + 1.9 per 256 elements (8 x 11008 x 4096 two rounds 50 us, 1024^3
+// four 39 us, 256^3 one 6.6 us). tiles(tm, tn): tiles of that size.
+template <class Tiles>
+static int plan_gemm_bf(vx_ctx ctx, uint32_t K, const Tiles& tiles, uint32_t pin) {
+    const double S = std::ceil(K / 32.0), cus = (double)ctx->num_cus;
+    double us[5];
+    for (int i = 0; i < 5; ++i) {
+        const double r = std::ceil((double)tiles(kBfRows[i], kBfCols[i]) / cus);
+        us[i] = i == BF_W    ? r * (8.0 + 2.55 * S)
+                : i == BF_N  ? r * (5.4 + 1.34 * S)
+                : i == BF_S2 ? r * (2.8 + 0.6 * S)
+                : i == BF_S  ? (r <= 1.0 ? 2.8 + 0.7 * S : r * (1.0 + 0.45 * S) + 0.1 * S + 1.0)
+                             : r * (2.0 + 1.9 * std::ceil(K / 256.0));
+    }
+    int cfg = BF_W;
+    for (int i = 1; i < 5; ++i)
+        if (us[i] < us[cfg]) cfg = i;
+    if (cfg == BF_KS || !pin) return cfg;
+    return pin == VX_GEMM_TILE_WIDE ? BF_W : pin == VX_GEMM_TILE_NARROW ? BF_N : us[BF_S2] < us[BF_S] ? BF_S2 : BF_S;
+}
+
+static int launch_gemm_bf(vx_ctx ctx, vx_stream stream, const vx_gemm_args& g, int cfg, uint32_t batch) {
+#define VX_B5(n) {K_vx_gemm_bf_##n##_w, K_vx_gemm_bf_##n##_n, K_vx_gemm_bf_##n##_s2, K_vx_gemm_bf_##n##_s, K_vx_gemm_bf_##n##_ks}
+    static const int tab[2][2][5] = {{VX_B5(kk), VX_B5(kx)}, {VX_B5(xk), VX_B5(xx)}};
+#undef VX_B5
+    // A / B with stride 1 along K: 16-byte loads along it (4-byte aligned: any row stride); else along M / N
+    const int k = tab[g.as[3] == 1 ? 0 : 1][g.bs[2] == 1 ? 0 : 1][cfg];
+    const uint32_t tm = kBfRows[cfg], tn = kBfCols[cfg];
+    // two buffers of a stage's terms (6 bytes an element) and a word; the K split: the waves' sums and 64 words
+    const size_t lds = cfg == BF_KS ? 8u * 4096u + 256u : (size_t)(tm + tn) * (cfg == BF_S2 ? 64u : 32u) * 12u + 16u;
+    // a grid holds fewer than 2^32 threads: at most 2^21 tiles per launch
+    const uint32_t sm = tm << 10, sn = tn << 11;
+    for (uint64_t m = 0; m < g.M; m += sm)
+        for (uint64_t n = 0; n < g.N; n += sn) {
+            vx_gemm_args a = g;
+            a.M = (uint32_t)std::min<uint64_t>(g.M - m, sm);
+            a.N = (uint32_t)std::min<uint64_t>(g.N - n, sn);
+            a.a = g.a + (int64_t)m * g.as[2];
+            a.b = g.b + (int64_t)n * g.bs[3];
+            a.c = g.c + (int64_t)m * g.cs[2] + (int64_t)n * g.cs[3];
+            a.tiles_m = (a.M + tm - 1) / tm;
+            a.tiles_n = (a.N + tn - 1) / tn;
+            const int s = launch(ctx, k, dim3(a.tiles_m * a.tiles_n, 1, batch), dim3(512), lds, stream, a);
+            if (s) return s;
+        }
+    return VX_OK;
+}
+
 static int run_gemm(vx_ctx ctx, vx_stream stream, const vx_mview* out, const vx_cview* lhs, const vx_cview* rhs,
                     int force, const vx_gemm_opts* opts = nullptr) {
     clear_error();
@@ -399,56 +459,48 @@ static int run_gemm(vx_ctx ctx, vx_stream stream, const vx_mview* out, const vx_
     if (p.route == VX_ROUTE_NAIVE) {
         return launch(ctx, K_vx_gemm_naive, dim3((p.N + 63) / 64, p.M, batch), dim3(64), 0, stream, a);
     }
-    a.tiles_m = (p.M + 127) / 128;
-    a.tiles_n = (p.N + 127) / 128;
     const int am = operand_mode(p.l, 3, 2, p.nb, p.nc);
     const int bm = operand_mode(p.r, 2, 3, p.nb, p.nc);
-    int k;
+    const uint32_t pin = opts ? opts->flags & (VX_GEMM_TILE_NARROW | VX_GEMM_TILE_WIDE | VX_GEMM_TILE_SMALL) : 0u;
+    const double cus = (double)ctx->num_cus;
+    auto tiles = [&](uint32_t tm, uint32_t tn) {
+        return (uint64_t)((p.M + (uint64_t)tm - 1) / tm) * ((p.N + (uint64_t)tn - 1) / tn) * batch;
+    };
+    // Few outputs: 32 x 32 tiles with K split over a workgroup's waves, where
+    // that is estimated fastest. This and the next choice come before the
+    // pinned tile shape, so that all pins give the same bits at any shape.
+    const int cfg = plan_gemm_bf(ctx, p.K, tiles, pin);
+    // A short K and not many outputs, rows contiguous and 16-byte aligned: the
+    // f32 MFMA kernels, whose tiles cost less to begin and to end (128 x 128 x
+    // 128, batch 32: 7.4 against 7.9 us; 2432 x 2368 x 96 20.1 / 21.0; 200 x
+    // 200 x 64, batch 40 10.3 / 14.1; but 1024 x 1024 x 64, batch 8 20.9 /
+    // 16.7 and 3040 x 384 x 160 13.0 / 12.5).
+    const bool shortk = p.K < 160u && am == 0 && bm != 2 && tiles(64, 64) <= 6ull * (uint64_t)ctx->num_cus;
+    if (cfg == BF_KS || !shortk) return launch_gemm_bf(ctx, stream, a, cfg, batch);
+    const uint64_t tn = tiles(128, 128), tw = tiles(128, 256), ts = tiles(64, 64);
     // Tile shape. 128 x 256 tiles (two resident workgroups per CU) instead of
     // 128 x 128 (three) when they fill the last round of resident workgroups
-    // clearly better: 4096^3 is 1024 narrow tiles, 1.33 rounds of 768, but 512
-    // wide ones, one round (B transposed 131 -> 137 TFLOP/s). 64 x 64 tiles
-    // when they spread over the CUs better than either, a CU taking
-    // ceil(tiles / CUs) of them, balance = (tiles / CUs) / that, the small
-    // kernel weighted 0.9 for its lower rate on large shapes (4096^3: 119 vs
-    // 131 TFLOP/s): 1024^3 28 -> 75, 1536^3 65 -> 80, 3072^3 96 -> 109. All
-    // give the same bits; VX_GEMM_TILE_* (vx_gemm_f32_ex) force one.
-    bool wide = false, small = false;
-    if (am == 0 && (bm == 0 || bm == 1)) {
-        const uint64_t tn = (uint64_t)a.tiles_m * a.tiles_n * batch;
-        const uint64_t tw = (uint64_t)a.tiles_m * ((p.N + 255) / 256) * batch;
-        const uint64_t ts = (uint64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * batch;
-        const uint64_t sn = 3ull * (uint64_t)ctx->num_cus, sw = 2ull * (uint64_t)ctx->num_cus;
-        const double en = (double)tn / (double)(((tn + sn - 1) / sn) * sn);
-        const double ew = (double)tw / (double)(((tw + sw - 1) / sw) * sw);
-        wide = ew > en + 0.05;
-        const double cus = (double)ctx->num_cus;
-        auto balance = [&](uint64_t t) { return ((double)t / cus) / std::ceil((double)t / cus); };
-        small = 0.9 * balance(ts) > std::max(balance(tn), balance(tw));
-        if (small) wide = false;
-        const uint32_t tf = opts ? opts->flags : 0u;
-        if (tf & (VX_GEMM_TILE_NARROW | VX_GEMM_TILE_WIDE | VX_GEMM_TILE_SMALL)) {
-            wide = (tf & VX_GEMM_TILE_WIDE) != 0;
-            small = (tf & VX_GEMM_TILE_SMALL) != 0;
-        }
+    // clearly better; 64 x 64 tiles when they spread over the CUs better than
+    // either, a CU taking ceil(tiles / CUs) of them, balance = (tiles / CUs) /
+    // that, the small kernel weighted 0.9 for its lower rate on large shapes.
+    // All give the same bits; VX_GEMM_TILE_* (vx_gemm_f32_ex) force one.
+    const uint64_t sn = 3ull * (uint64_t)ctx->num_cus, sw = 2ull * (uint64_t)ctx->num_cus;
+    const double en = (double)tn / (double)(((tn + sn - 1) / sn) * sn);
+    const double ew = (double)tw / (double)(((tw + sw - 1) / sw) * sw);
+    auto balance = [&](uint64_t t) { return ((double)t / cus) / std::ceil((double)t / cus); };
+    bool small = 0.9 * balance(ts) > std::max(balance(tn), balance(tw));
+    bool wide = !small && ew > en + 0.05;
+    if (pin) {
+        wide = pin == VX_GEMM_TILE_WIDE;
+        small = pin == VX_GEMM_TILE_SMALL;
     }
-    if (small) {
-        a.tiles_m = (p.M + 63) / 64;
-        a.tiles_n = (p.N + 63) / 64;
-        k = bm == 1 ? K_vx_gemm_mfma_kx_s : K_vx_gemm_mfma_kk_s;
-    } else if (wide) {
-        a.tiles_n = (p.N + 255) / 256;
-        k = bm == 1 ? K_vx_gemm_mfma_kx_w : K_vx_gemm_mfma_kk_w;
-    } else if (am == 0 && bm == 1) k = K_vx_gemm_mfma_kx;
-    else if (am == 0 && bm == 0) k = K_vx_gemm_mfma_kk;
-    else if (am == 1 && bm == 1) k = K_vx_gemm_mfma_xx;
-    else if (am == 1 && bm == 0) k = K_vx_gemm_mfma_xk;
-    else if (am == 0) k = K_vx_gemm_mfma_kg;
-    else if (bm == 1) k = K_vx_gemm_mfma_gx;
-    else k = K_vx_gemm_mfma_gg;
-    const uint64_t tiles = (uint64_t)a.tiles_m * a.tiles_n;
-    if (tiles > 0x7FFFFFFFull) return fail(VX_ERR_UNSUPPORTED, "too many output tiles");
-    return launch(ctx, k, dim3((uint32_t)tiles, 1, batch), dim3(VX_WG), 0, stream, a);
+    const uint32_t tm = small ? 64u : 128u, tnn = small ? 64u : wide ? 256u : 128u;
+    a.tiles_m = (p.M + tm - 1) / tm;
+    a.tiles_n = (p.N + tnn - 1) / tnn;
+    const int k = small  ? (bm == 1 ? K_vx_gemm_mfma_kx_s : K_vx_gemm_mfma_kk_s)
+                  : wide ? (bm == 1 ? K_vx_gemm_mfma_kx_w : K_vx_gemm_mfma_kk_w)
+                         : (bm == 1 ? K_vx_gemm_mfma_kx : K_vx_gemm_mfma_kk);
+    return launch(ctx, k, dim3(a.tiles_m * a.tiles_n, 1, batch), dim3(VX_WG), 0, stream, a);
 }
 
 // ------------------------------------------------------------ quant gemv
