@@ -996,6 +996,80 @@ __device__ __forceinline__ void vx_dequant(const vx_gemv_args& a) {
     for (int i = 0; i < 32; ++i) op[(int64_t)i * a.ys_b] = o[i];
 }
 
+// The same for an output with stride 1 along k: 8 threads per 32-weight group,
+// thread i decoding weights 4i..4i+3 from one dword, so that a wave stores 1
+// KB of consecutive output per instruction (16 bytes a lane, 4-byte aligned).
+// The kernel above stores 4 bytes a lane, 128 bytes apart, which is why it
+// stays for other strides only. 14336 x 4096, that one / this one: Q4_0 254 / 40
+// us, Q8_0 261 / 55, Q4_K 255 / 41 (6.6 TB/s of blocks read and floats written:
+// bound by memory).
+// A workgroup takes VX_DQ_GROUPS consecutive groups of the flattened (row,
+// group) sequence, a thread VX_DQ_U of them, every load ahead of the first
+// store. W may have any alignment.
+#define VX_DQ_U 4
+#define VX_DQ_GROUPS (VX_DQ_U * VX_WG / 8u)
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
+typedef uint16_t u16_a1 __attribute__((aligned(1)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int QT>
+__device__ __forceinline__ void vx_dequant_rows(const vx_gemv_args& a) {
+    const uint32_t ng = a.K / 32u, i = threadIdx.x & 7u;
+    const uint64_t g0 = (uint64_t)blockIdx.x * VX_DQ_GROUPS, end = (uint64_t)a.M * ng;
+    const uint32_t m0 = (uint32_t)(g0 / ng), k0 = (uint32_t)(g0 - (uint64_t)m0 * ng);  // uniform
+    uint32_t q[VX_DQ_U], h[VX_DQ_U], s1[VX_DQ_U], s2[VX_DQ_U], s3[VX_DQ_U], kb[VX_DQ_U], m[VX_DQ_U];
+#pragma unroll
+    for (int u = 0; u < VX_DQ_U; ++u) {
+        // (past the end: the last group again, not stored)
+        const uint32_t o = min((threadIdx.x >> 3) + (uint32_t)u * (VX_WG / 8u), (uint32_t)min(end - 1u - g0, (uint64_t)VX_DQ_GROUPS));
+        const uint32_t t = k0 + o;  // (K < 2^32 and o small: no carry)
+        m[u] = m0 + t / ng;
+        kb[u] = t % ng;
+        const uint8_t* row = a.w + (uint64_t)m[u] * a.row_stride;
+        if constexpr (QT == VX_Q4_0) {
+            const uint8_t* p = row + 18ull * kb[u];
+            h[u] = *(const u16_a1*)p;
+            q[u] = *(const u32_a1*)(p + 2 + 4u * (i & 3u));
+        } else if constexpr (QT == VX_Q8_0) {
+            const uint8_t* p = row + 34ull * kb[u];
+            h[u] = *(const u16_a1*)p;
+            q[u] = *(const u32_a1*)(p + 2 + 4u * i);
+        } else {
+            const uint8_t* p = row + 144ull * (kb[u] >> 3);
+            h[u] = *(const u32_a1*)p;
+            s1[u] = *(const u32_a1*)(p + 4);
+            s2[u] = *(const u32_a1*)(p + 8);
+            s3[u] = *(const u32_a1*)(p + 12);
+            q[u] = *(const u32_a1*)(p + 16 + 32u * ((kb[u] & 7u) >> 1) + 4u * i);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < VX_DQ_U; ++u) {
+        if (g0 + (threadIdx.x >> 3) + (uint32_t)u * (VX_WG / 8u) >= end) continue;
+        float o[4];
+        if constexpr (QT == VX_Q4_0) {
+            const float d = vx_f16_to_f32(h[u]);
+            const uint32_t n = (i < 4u ? q[u] : q[u] >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (float)((int)((n >> (8 * e)) & 15u) - 8) * d;
+        } else if constexpr (QT == VX_Q8_0) {
+            const float d = vx_f16_to_f32(h[u]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = d * (float)(int8_t)((q[u] >> (8 * e)) & 0xFFu);
+        } else {
+            uint32_t sc0, mn0, sc1, mn1;
+            vx_q4k_scales(s1[u], s2[u], s3[u], (kb[u] & 7u) >> 1, sc0, mn0, sc1, mn1);
+            const bool hi = kb[u] & 1u;
+            const float ds = vx_f16_to_f32(h[u]) * (float)(hi ? sc1 : sc0);
+            const float mm = vx_f16_to_f32(h[u] >> 16) * (float)(hi ? mn1 : mn0);
+            const uint32_t n = (hi ? q[u] >> 4 : q[u]) & 0x0F0F0F0Fu;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = __fsub_rn(__fmul_rn(ds, (float)((n >> (8 * e)) & 15u)), mm);
+        }
+        *(f32x4_a4*)(a.y + (int64_t)m[u] * a.ys_m + (int64_t)(32ull * kb[u] + 4u * i)) = f32x4_a4{o[0], o[1], o[2], o[3]};
+    }
+}
+
 // Arguments of the persistent batch-1 kernels (and of the read probe and the
 // launch floor, which mirror them). What a wave needs before its first x and
 // weight requests (W, x, the row stride, M, the units per row, the grid size
@@ -1093,6 +1167,10 @@ __device__ __forceinline__ vx_gemv_args vx_b1_args(const uint8_t* w, const float
     extern "C" __global__ __launch_bounds__(VX_WG) void vx_dequant_##QN(vx_gemv_args a) {          \
         vx_args_fetch(a);                                                                           \
         vx_dequant<QT>(a);                                                                          \
+    }                                                                                               \
+    extern "C" __global__ __launch_bounds__(VX_WG) void vx_dequant_rows_##QN(vx_gemv_args a) {     \
+        vx_args_fetch(a);                                                                           \
+        vx_dequant_rows<QT>(a);                                                                     \
     }
 
 VX_GEMV_ALL(VX_Q4_0, q4_0)

@@ -577,8 +577,12 @@ static int generic_kernel(uint32_t qt) {
     return qt == VX_Q4_0 ? K_vx_gemv_generic_q4_0 : qt == VX_Q8_0 ? K_vx_gemv_generic_q8_0 : K_vx_gemv_generic_q4_k;
 }
 
-static int dequant_kernel(uint32_t qt) {
-    return qt == VX_Q4_0 ? K_vx_dequant_q4_0 : qt == VX_Q8_0 ? K_vx_dequant_q8_0 : K_vx_dequant_q4_k;
+// rows: output with stride 1 along K
+static int dequant_kernel(uint32_t qt, bool rows) {
+    static const int tab[3][2] = {{K_vx_dequant_q4_0, K_vx_dequant_rows_q4_0},
+                                  {K_vx_dequant_q8_0, K_vx_dequant_rows_q8_0},
+                                  {K_vx_dequant_q4_k, K_vx_dequant_rows_q4_k}};
+    return tab[q_index(qt)][rows ? 1 : 0];
 }
 
 // Rows per wave for batch 1: the largest R whose grid still gives every
@@ -1319,8 +1323,12 @@ static int run_dequant(vx_ctx ctx, vx_stream stream, const vx_mview* out, const 
     a.ys_b = co.l.stride[3];
     a.M = w->rows;
     a.K = w->cols;
-    return launch(ctx, dequant_kernel(w->qtype), dim3((uint32_t)((groups + VX_WG - 1) / VX_WG)), dim3(VX_WG), 0,
-                  stream, a);
+    // stride 1 along K: 128 groups per workgroup (fewer than 2^24 of them: a
+    // grid holds fewer than 2^32 threads), else a group per thread
+    const bool rows = a.ys_b == 1 && groups < (1ull << 31);
+    const uint64_t per = rows ? 128u : VX_WG;
+    return launch(ctx, dequant_kernel(w->qtype, rows), dim3((uint32_t)((groups + per - 1) / per)), dim3(VX_WG), 0, stream,
+                  a);
 }
 
 }  // namespace vx
