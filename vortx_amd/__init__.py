@@ -35,6 +35,18 @@ __all__ = ["TensorLayout", "layout_extent", "XQ", "xq_size", "Gemm", "QuantGemv"
 lib()
 
 
+# Calls with plain torch tensors build their views in C (csrc/vx_pycall.cpp);
+# those functions return None for anything else, which then takes the ctypes
+# path below.
+from . import _pycall  # noqa: E402
+
+_ADDR = {name: C.cast(getattr(lib(), name), C.c_void_p).value
+         for name in ("vx_gemm_f32", "vx_gemm_f32_ex", "vx_gemv_q_ex", "vx_gemv_q_ws", "vx_dequantize", "vx_quantize",
+                      "vx_contiguous")}
+_GEMM, _GEMM_EX = _ADDR["vx_gemm_f32"], _ADDR["vx_gemm_f32_ex"]
+_GEMV_EX, _GEMV_WS = _ADDR["vx_gemv_q_ex"], _ADDR["vx_gemv_q_ws"]
+
+
 # ---------------------------------------------------------------- layout
 @dataclass(frozen=True)
 class TensorLayout:
@@ -163,6 +175,7 @@ class _Context:
         h = C.c_void_p()
         check(lib().vx_init(device, C.byref(h)))
         self._h = h
+        self._ctx = h.value  # 0 after close()
         self.device = device
         n = C.c_int()
         check(lib().vx_device_info(h, None, C.byref(n)))
@@ -172,6 +185,7 @@ class _Context:
         if getattr(self, "_h", None):
             lib().vx_destroy(self._h)
             self._h = None
+            self._ctx = 0
 
     def __del__(self):
         try:
@@ -193,7 +207,11 @@ class Gemm(_Context):
         check(fn(self._h, _stream(stream), C.byref(o), C.byref(l), C.byref(r)))
 
     def dispatch(self, out, lhs, rhs, stream=None) -> None:
-        self._call(lib().vx_gemm_f32, out, lhs, rhs, stream)
+        st = _pycall.gemm(_GEMM, self._ctx, stream, out, lhs, rhs)
+        if st is None:
+            self._call(lib().vx_gemm_f32, out, lhs, rhs, stream)
+        elif st:
+            check(st)
 
     def dispatch_ex(self, out, lhs, rhs, alpha: float = 1.0, beta: float = 0.0, broadcast: bool = False,
                     tile: str = "auto", stream=None) -> None:
@@ -202,10 +220,15 @@ class Gemm(_Context):
         are reused along out's (src/shapes.rs:346-391 semantics). ``tile``:
         "narrow" / "wide" / "small" pins the MFMA kernels' 128 x 128 / 256 x 128 /
         64 x 64 output tiles (same bits every way), "auto" lets the library choose."""
-        o, l, r = _view_of(out, True), _view_of(lhs, False), _view_of(rhs, False)
         flags = (_ffi.VX_GEMM_BROADCAST if broadcast else 0) | {"auto": 0, "narrow": _ffi.VX_GEMM_TILE_NARROW,
                                                                  "wide": _ffi.VX_GEMM_TILE_WIDE,
                                                                  "small": _ffi.VX_GEMM_TILE_SMALL}[tile]
+        st = _pycall.gemm(_GEMM_EX, self._ctx, stream, out, lhs, rhs, alpha, beta, flags)
+        if st is not None:
+            if st:
+                check(st)
+            return
+        o, l, r = _view_of(out, True), _view_of(lhs, False), _view_of(rhs, False)
         opts = _ffi.VxGemmOpts(alpha, beta, flags, 0)
         check(lib().vx_gemm_f32_ex(self._h, _stream(stream), C.byref(o), C.byref(l), C.byref(r), C.byref(opts)))
 
@@ -263,6 +286,15 @@ class QWeight:
         w.reserved = 0
         w.row_stride_bytes = self.row_stride
         return w
+
+
+def _setup_pycall():
+    import torch
+    _pycall.setup(QWeight, torch.Tensor, torch.float32, getattr(torch._C, "_cuda_getCurrentRawStream", None),
+                  getattr(torch._C, "_cuda_getDevice", None))
+
+
+_setup_pycall()
 
 
 def xq_size(K: int, B: int) -> int:
@@ -351,8 +383,13 @@ class QuantGemv(_Context):
         ``workspace_size(w, B)`` bytes (vx_gemv_q_ws), where batched shapes
         split x when the GEMV kernel cannot split it itself; without one
         those shapes keep x in f32 (or, with ``x_int8``, raise)."""
-        yv, xv, wc = _view_of(y, True), _view_of(x, False), w._c()
         flags = (_ffi.VX_GEMV_X_F32 if x_f32 else 0) | (_ffi.VX_GEMV_X_INT8 if x_int8 else 0)
+        st = _pycall.gemv(_GEMV_EX, _GEMV_WS, self._ctx, stream, y, w, x, flags, workspace)
+        if st is not None:
+            if st:
+                check(st)
+            return
+        yv, xv, wc = _view_of(y, True), _view_of(x, False), w._c()
         if workspace is None:
             check(lib().vx_gemv_q_ex(self._h, _stream(stream), C.byref(yv), C.byref(wc), C.byref(xv), flags))
             return
@@ -381,10 +418,20 @@ class QuantGemv(_Context):
     def quantize(self, out: "QWeight", x, stream=None) -> None:
         """Write the blocks of ``out`` from the f32 [rows, cols] view ``x``
         (ggml's reference quantizers; see include/vortx_hip.h vx_quantize)."""
+        st = _pycall.quantize(_ADDR["vx_quantize"], self._ctx, stream, out, x)
+        if st is not None:
+            if st:
+                check(st)
+            return
         xv, wc = _view_of(x, False), out._c()
         check(lib().vx_quantize(self._h, _stream(stream), C.byref(wc), C.byref(xv)))
 
     def dequantize(self, out, w: QWeight, stream=None) -> None:
+        st = _pycall.dequantize(_ADDR["vx_dequantize"], self._ctx, stream, out, w)
+        if st is not None:
+            if st:
+                check(st)
+            return
         ov, wc = _view_of(out, True), w._c()
         check(lib().vx_dequantize(self._h, _stream(stream), C.byref(ov), C.byref(wc)))
 
@@ -397,6 +444,12 @@ class Contiguous(_Context):
     the view's own offset is ignored, as in the reference."""
 
     def launch(self, out, tensor, offset=None, stream=None) -> None:
+        if offset is None:  # (with one, the raw buffer and the view's offset matter apart)
+            st = _pycall.contiguous(_ADDR["vx_contiguous"], self._ctx, stream, out, tensor)
+            if st is not None:
+                if st:
+                    check(st)
+                return
         import torch
         ov, tv = _view_of(out, True, any4=True), _view_of(tensor, False, any4=True)
         off = None

@@ -6,7 +6,8 @@ Steps (no cmake):
   2. an assembler stub that .incbin's those code objects, so the shared
      library carries them and vx_init can hipModuleLoadData them;
   3. g++ for the host sources (HIP runtime API only), linked against
-     libamdhip64.
+     libamdhip64;
+  4. g++ for the CPython extension with the binding's fast calls (_pycall.so).
 
 Every call recompiles everything (a build check, not an incremental build).
 """
@@ -17,12 +18,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 INCLUDE = os.path.join(os.path.dirname(PKG), "include")  # the public C ABI header
 CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libvortx_hip.so")
+PYCALL = os.path.join(PKG, "_pycall.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 
@@ -81,6 +84,11 @@ def build(verbose: bool = False) -> str:
            f"-L{ROCM}/lib", "-lamdhip64", f"-Wl,-rpath,{ROCM}/lib", "-o", tmp]
     _run(cmd)
     os.replace(tmp, LIB)
+    tmp = PYCALL + ".tmp"
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-cast-function-type",
+          "-Wno-missing-field-initializers", f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}",
+          os.path.join(CSRC, "vx_pycall.cpp"), "-o", tmp])
+    os.replace(tmp, PYCALL)
     if verbose:
         print(f"built {LIB}")
     return LIB
