@@ -1607,27 +1607,6 @@ __device__ __forceinline__ void vx_gemv_xq(const vx_gemv_xq_args& a) {
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if constexpr (FX) {
-        // (issuing the ring between the x loads and the split arithmetic, to
-        // overlap the two, measured 8-13 % slower: as with x levels, weight
-        // requests ahead of a CU's x requests delay x more than they gain)
-        pass_split(0u);
-        ring_prologue();
-    } else {
-        // x requests first; a bare barrier puts every x request of the CU
-        // ahead of every weight request; then the ring, and only then the
-        // wait for this wave's x (the scales go to LDS). Measured against
-        // waiting for x before issuing the ring (graph-replayed, same box):
-        // Q4_0 4096x11008 B = 8 10.2 -> 9.5 us, 11008x4096 B = 8 9.5 -> 8.9 us,
-        // Q4_K 32000x4096 B = 16 26.5 -> 25.5 us, 14336x4096 B = 16 even.
-        pass_loads(0u);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        ring_prologue();
-        pass_publish(0u);
-    }
-
     float acc[NCG][2];
 #pragma unroll
     for (int h = 0; h < NCG; ++h) acc[h][0] = acc[h][1] = 0.f;
@@ -1660,6 +1639,50 @@ __device__ __forceinline__ void vx_gemv_xq(const vx_gemv_xq_args& a) {
         }
         __syncthreads();
     };
+
+    if constexpr (!MP) {
+        if ((uint32_t)XI * slot >= ipr) {  // wave-uniform
+            // K has no item for this wave (K < 4096 with one item a wave): it
+            // parks zeros and meets the others. Splitting and reducing a
+            // clamped item instead takes VALU issue and L2 requests from the
+            // waves that have one (us, before / after, graph-replayed: Q4_0
+            // 1536^2 B = 4 5.2 / 4.5, B = 8 6.6 / 5.3; 14336x2048 B = 8 10.9 /
+            // 8.1; Q8_0 14336x2048 B = 2 12.7 / 8.4; Q4_K 7424x2560 B = 16
+            // 9.1 / 8.5; with no idle wave, 4096^2 to 32000x4096, within 3 %
+            // either way).
+            if constexpr (!FX) __builtin_amdgcn_s_barrier();  // the others' bare barrier
+            for (uint32_t w = 0, f = 0; w < nwork; ++w) {
+                float* rb = red + (w % RMAX) * TILE_F + slot * CP * 16u;
+#pragma unroll
+                for (uint32_t e = 0; e < CP * 16u / 64u; ++e) rb[lane + 64u * e] = 0.f;
+                if (w + 1u == nwork || w + 1u - f == RMAX) {
+                    flush(f, w);
+                    f = w + 1u;
+                }
+            }
+            return;
+        }
+    }
+    if constexpr (FX) {
+        // (issuing the ring between the x loads and the split arithmetic, to
+        // overlap the two, measured 8-13 % slower: as with x levels, weight
+        // requests ahead of a CU's x requests delay x more than they gain)
+        pass_split(0u);
+        ring_prologue();
+    } else {
+        // x requests first; a bare barrier puts every x request of the CU
+        // ahead of every weight request; then the ring, and only then the
+        // wait for this wave's x (the scales go to LDS). Measured against
+        // waiting for x before issuing the ring (graph-replayed, same box):
+        // Q4_0 4096x11008 B = 8 10.2 -> 9.5 us, 11008x4096 B = 8 9.5 -> 8.9 us,
+        // Q4_K 32000x4096 B = 16 26.5 -> 25.5 us, 14336x4096 B = 16 even.
+        pass_loads(0u);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        ring_prologue();
+        pass_publish(0u);
+    }
 
     uint32_t wflush = 0;  // first tile-work not yet written to y
     auto tile_work = [&](uint32_t w, int u, bool refill) {
