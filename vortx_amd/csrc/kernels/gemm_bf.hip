@@ -13,7 +13,7 @@
 // -> 650 us (212 TFLOP/s of f32 work, 1270 of bf16; a bf16 product of that size
 // by the vendor's library 1370 on this card), 4096 x 11008 x 4096 2720 -> 1870,
 // 1024^3 26 -> 23.5, 1000 x 1111 x 777 with odd strides 119 -> 28, 8 x 11008 x
-// 4096 154 -> 53 (K split), 64 x 64 x 4096 394 -> 25.5 (K split). The large
+// 4096 154 -> 44 (K split), 64 x 64 x 4096 394 -> 13 (K split). The large
 // shapes are bound by the matrix cores and the card's power, the smaller ones
 // by the stages' serial steps (load, convert, store, barrier, read, multiply)
 // with one workgroup per CU.
@@ -24,11 +24,19 @@
 #include "vx_bf16.hpp"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // Operand access: "x" is the non-K dimension (M for A, N for B).
 #define MODE_K 0  // stride 1 along K
 #define MODE_X 1  // any strides; best with stride 1 along x
+
+// Workgroup ids are dealt round robin to 8 XCDs: the id's place when each XCD
+// takes a contiguous run of tiles (any number of them: with runs only for
+// multiples of 8, 21 x 4588 x 1991 in 574 tiles took 35 us instead of 20.6).
+__device__ __forceinline__ uint32_t vx_xcd_order(uint32_t bid, uint32_t nt) {
+    return (bid & 7u) * (nt >> 3) + min(bid & 7u, nt & 7u) + (bid >> 3);
+}
 
 __device__ __forceinline__ void vx_epilogue(float* c, float acc, float alpha, float beta) {
     *c = beta == 0.f ? alpha * acc : alpha * acc + beta * *c;
@@ -131,8 +139,7 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
     // 8), then walked in groups of 8 tile rows, so that an XCD's resident
     // tiles share panels of A and B in its L2.
     const uint32_t nt = p.tiles_m * p.tiles_n;
-    uint32_t bid = blockIdx.x;
-    if ((nt & 7u) == 0) bid = (bid & 7u) * (nt >> 3) + (bid >> 3);
+    const uint32_t bid = vx_xcd_order(blockIdx.x, nt);
     const uint32_t group = 8u * p.tiles_n;
     const uint32_t first_m = (bid / group) * 8u;
     const uint32_t gsize = min(p.tiles_m - first_m, 8u);
@@ -421,8 +428,7 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
     const uint32_t t = threadIdx.x, lane = t & 63u, n = lane & 31u, g = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint32_t nt = p.tiles_m * p.tiles_n;
-    uint32_t bid = blockIdx.x;  // tiles that share columns of B follow each other on one XCD
-    if ((nt & 7u) == 0) bid = (bid & 7u) * (nt >> 3) + (bid >> 3);
+    const uint32_t bid = vx_xcd_order(blockIdx.x, nt);  // tiles that share columns of B follow each other on one XCD
     const uint32_t m0 = bid % p.tiles_m * 32u, n0 = bid / p.tiles_m * 32u;
     const uint32_t z = blockIdx.z;
     const uint32_t bn = z / p.batch_c, bc = z % p.batch_c;
@@ -511,6 +517,127 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
     }
 }
 
+// 16 x 16 tiles on 16 x 16 x 32 products, K split over the 8 waves as above.
+// Against 32 x 32 tiles, four times the workgroups, and few enough registers
+// for two or three on a CU: the shapes with about as many 32 x 32 tiles as CUs,
+// or fewer, ran at the pace of one workgroup on some of the CUs (or of a second
+// round on a few). Each operand is read and split once per 16 outputs of the
+// other, so it loses where 32 x 32 tiles fill the card. Graph-replayed, us, 32 x
+// 32 / 16 x 16: 8 x 11008 x 4096 B [N, K] 52.7 / 44.1, 16 x 4096 x 4096 28.4 /
+// 19.5, 23 x 1989 x 5973 34.8 / 22.0, 96 x 64 x 3776 A [K, M] 24.9 / 13.1, 256^3
+// 5.3 / 4.1; but 30 x 16384 x 2048 41 / 73, 512^3 8.0 / 12.2. Tried: 4 or 16
+// waves (44.4, 47.2 us on the first), three or four chunks ahead (no gain), 32 x
+// 16 tiles (46.3; 31 x 4096 x 4096 25.6 against 33.7 and 34.5, the only size
+// where they won).
+template <int MODE>
+struct vx_strip {  // one operand's 32 k of lane (n, g)'s x: elements 8g..8g+7
+    float r[8];
+    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0, uint32_t g) {
+        const uint32_t k = k0 + 8u * g;
+        if constexpr (MODE == MODE_K) {
+            const f32x4_a4 a = *(const f32x4_a4*)(p + k), b = *(const f32x4_a4*)(p + k + 4);
+            r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+            r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r[j] = p[(int64_t)(k + (uint32_t)j) * sk];
+        }
+    }
+    __device__ __forceinline__ void load_tail(const float* p, int64_t sk, uint32_t k0, uint32_t g, uint32_t K) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t k = k0 + 8u * g + (uint32_t)j, kc = min(k, K - 1u);
+            const float e = p[MODE == MODE_K ? (int64_t)kc : (int64_t)kc * sk];  // (clamped: no branches between the loads)
+            r[j] = k < K ? e : 0.f;
+        }
+    }
+};
+
+template <int AM, int BM>
+__device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
+    constexpr uint32_t NWV = 8;
+    const uint32_t t = threadIdx.x, lane = t & 63u, n = lane & 15u, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t bid = vx_xcd_order(blockIdx.x, p.tiles_m * p.tiles_n);  // tiles that share columns of B on one XCD
+    const uint32_t m0 = bid % p.tiles_m * 16u, n0 = bid / p.tiles_m * 16u;
+    const uint32_t z = blockIdx.z;
+    const uint32_t bn = z / p.batch_c, bc = z % p.batch_c;
+    const float* A = p.a + bn * p.as[0] + bc * p.as[1];
+    const float* B = p.b + bn * p.bs[0] + bc * p.bs[1];
+    float* C = p.c + bn * p.cs[0] + bc * p.cs[1];
+    const float* pa = A + (int64_t)min(m0 + n, p.M - 1u) * p.as[2];
+    const float* pb = B + (int64_t)min(n0 + n, p.N - 1u) * p.bs[3];
+
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // even and odd chunks
+    float ma = 0.f, mb = 0.f;  // the largest |element| seen
+    auto mult = [&](const vx_strip<AM>& a, const vx_strip<BM>& b, int par) {
+        u32x4 ta[3], tb[3];
+        vx_split8_rne(a.r, ta);
+        vx_split8_rne(b.r, tb);
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            ma = fmaxf(fmaxf(__builtin_fabsf(a.r[j]), __builtin_fabsf(a.r[j + 1])), ma);
+            mb = fmaxf(fmaxf(__builtin_fabsf(b.r[j]), __builtin_fabsf(b.r[j + 1])), mb);
+        }
+        constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};  // smallest products first
+#pragma unroll
+        for (int e = 0; e < 6; ++e)
+            acc[par] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ta[TA[e]]),
+                                                               __builtin_bit_cast(bf16x8, tb[TB[e]]), acc[par], 0, 0, 0);
+    };
+    const uint32_t nck = p.K / 32u;  // whole chunks
+    if (wave < nck) {
+        vx_strip<AM> a[2];
+        vx_strip<BM> b[2];
+        const uint32_t last = (nck - 1u - wave) / NWV * NWV + wave;  // this wave's last chunk
+        auto load = [&](int d, uint32_t c) {
+            a[d].load(pa, p.as[3], min(c, last) * 32u, g);
+            b[d].load(pb, p.bs[2], min(c, last) * 32u, g);
+        };
+        load(0, wave);
+        load(1, wave + NWV);
+        uint32_t c = wave;
+        for (; c + NWV <= last; c += 2u * NWV) {
+            __builtin_amdgcn_sched_barrier(0);  // (as in vx_gemm_bf_ks)
+            mult(a[0], b[0], 0);
+            load(0, c + 2u * NWV);
+            __builtin_amdgcn_sched_barrier(0);
+            mult(a[1], b[1], 1);
+            load(1, c + 3u * NWV);
+        }
+        if (c <= last) mult(a[0], b[0], 0);
+    }
+    if (p.K % 32u != 0u && wave == nck % NWV) {
+        vx_strip<AM> a;
+        vx_strip<BM> b;
+        a.load_tail(pa, p.as[3], nck * 32u, g, p.K);
+        b.load_tail(pb, p.bs[2], nck * 32u, g, p.K);
+        mult(a, b, 1);
+    }
+    // red[wave][v][lane], and the largest elements of the tile's rows of A and columns of B
+    float* red = (float*)vx_bf_lds;
+    uint32_t* mx = (uint32_t*)(red + NWV * 256u);
+    if (t < 32u) mx[t] = 0u;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave * 256u + (uint32_t)v * 64u + lane] = acc[0][v] + acc[1][v];
+    __syncthreads();
+    atomicMax(&mx[n], __float_as_uint(ma));
+    atomicMax(&mx[16u + n], __float_as_uint(mb));
+    __syncthreads();
+    if (t >= 256u) return;
+    float s = red[t];
+#pragma unroll
+    for (uint32_t w = 1; w < NWV; ++w) s += red[w * 256u + t];
+    const uint32_t rt = 4u * ((t & 63u) >> 4) + (t >> 6), ct = t & 15u;
+    const uint32_t row = m0 + rt, col = n0 + ct;
+    if (row >= p.M || col >= p.N) return;
+    const float rm = __uint_as_float(mx[rt]), cm = __uint_as_float(mx[16u + ct]);
+    const bool tiny = (rm * cm < 0x1p-80f || fminf(rm, cm) < 0x1p-109f) && rm > 0.f && cm > 0.f;
+    if (!(__builtin_fabsf(s) < __builtin_inff()) || tiny)
+        s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
+    vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+}
+
 // 256 x 128 tiles (8 waves of 64 x 64), 128 x 128 (2 x 4 waves of 64 x 64) and
 // 64 x 64 (2 x 4 waves of 32 x 32): _s up to three workgroups per CU, _s2 one,
 // with half the barriers.
@@ -527,6 +654,10 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
     extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 3)))              \
     void vx_gemm_bf_##NAME##_ks(vx_gemm_args p) {                                                        \
         vx_gemm_bf_ks<AM, BM>(p);                                                                        \
+    }                                                                                                    \
+    extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 6)))              \
+    void vx_gemm_bf_##NAME##_k16(vx_gemm_args p) {                                                       \
+        vx_gemm_bf_k16<AM, BM>(p);                                                                       \
     }
 VX_GEMM_BF(MODE_K, MODE_X, kx)
 VX_GEMM_BF(MODE_K, MODE_K, kk)

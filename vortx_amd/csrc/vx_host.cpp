@@ -327,8 +327,8 @@ static int operand_mode(const Canon& c, int kdim, int xdim, uint32_t nb, uint32_
 }
 
 // The bf16 matrix-core GEMM (gemm_bf.hip): tile shapes and the K split.
-enum BfCfg { BF_W = 0, BF_N = 1, BF_S2 = 2, BF_S = 3, BF_KS = 4 };
-static const uint32_t kBfRows[5] = {256, 128, 64, 64, 32}, kBfCols[5] = {128, 128, 64, 64, 32};
+enum BfCfg { BF_W = 0, BF_N = 1, BF_S2 = 2, BF_S = 3, BF_KS = 4, BF_K16 = 5 };
+static const uint32_t kBfRows[6] = {256, 128, 64, 64, 32, 16}, kBfCols[6] = {128, 128, 64, 64, 32, 16};
 // Choice by estimated time in us, rounds of resident workgroups times what a
 // round costs: a fixed part (first loads, last stores) and one per 32 elements
 // of K. Measured (graph-replayed): 256 x 128 tiles 8 + 2.55 (4096^3 2 rounds
@@ -337,35 +337,39 @@ static const uint32_t kBfRows[5] = {256, 128, 64, 64, 32}, kBfCols[5] = {128, 12
 // 0.6 (1024^3 one round 23.5 us), with short ones, three per CU, per tile of a
 // CU 1 + 0.45 (1000 x 1111 x 777 31 us, against 42 with long stages); the K
 // split 2 + 1.9 per 256 elements (8 x 11008 x 4096 two rounds 50 us, 1024^3
-// four 39 us, 256^3 one 6.6 us). tiles(tm, tn): tiles of that size.
+// four 39 us, 256^3 one 6.6 us); in 16 x 16 tiles, several on a CU, 2.2 and per
+// tile of a CU 0.4 + 1 per 256 (8 x 11008 x 4096 44 us, 512^3 12.2, 256^3 4.1,
+// 16 x 4096 x 4096 17.5 to 19.5). tiles(tm, tn): tiles of that size.
 template <class Tiles>
 static int plan_gemm_bf(vx_ctx ctx, uint32_t K, const Tiles& tiles, uint32_t pin) {
     const double S = std::ceil(K / 32.0), cus = (double)ctx->num_cus;
-    double us[5];
-    for (int i = 0; i < 5; ++i) {
-        const double r = std::ceil((double)tiles(kBfRows[i], kBfCols[i]) / cus);
+    double us[6];
+    for (int i = 0; i < 6; ++i) {
+        const double t = (double)tiles(kBfRows[i], kBfCols[i]) / cus, r = std::ceil(t);
         us[i] = i == BF_W    ? r * (8.0 + 2.55 * S)
                 : i == BF_N  ? r * (5.4 + 1.34 * S)
                 : i == BF_S2 ? r * (2.8 + 0.6 * S)
                 : i == BF_S  ? (r <= 1.0 ? 2.8 + 0.7 * S : r * (1.0 + 0.45 * S) + 0.1 * S + 1.0)
-                             : r * (2.0 + 1.9 * std::ceil(K / 256.0));
+                : i == BF_KS ? r * (2.0 + 1.9 * std::ceil(K / 256.0))
+                             : 2.2 + std::max(t, 1.0) * (0.4 + K / 256.0);
     }
     int cfg = BF_W;
-    for (int i = 1; i < 5; ++i)
+    for (int i = 1; i < 6; ++i)
         if (us[i] < us[cfg]) cfg = i;
-    if (cfg == BF_KS || !pin) return cfg;
+    if (cfg >= BF_KS || !pin) return cfg;
     return pin == VX_GEMM_TILE_WIDE ? BF_W : pin == VX_GEMM_TILE_NARROW ? BF_N : us[BF_S2] < us[BF_S] ? BF_S2 : BF_S;
 }
 
 static int launch_gemm_bf(vx_ctx ctx, vx_stream stream, const vx_gemm_args& g, int cfg, uint32_t batch) {
-#define VX_B5(n) {K_vx_gemm_bf_##n##_w, K_vx_gemm_bf_##n##_n, K_vx_gemm_bf_##n##_s2, K_vx_gemm_bf_##n##_s, K_vx_gemm_bf_##n##_ks}
-    static const int tab[2][2][5] = {{VX_B5(kk), VX_B5(kx)}, {VX_B5(xk), VX_B5(xx)}};
-#undef VX_B5
+#define VX_B6(n) {K_vx_gemm_bf_##n##_w, K_vx_gemm_bf_##n##_n, K_vx_gemm_bf_##n##_s2, K_vx_gemm_bf_##n##_s, K_vx_gemm_bf_##n##_ks, K_vx_gemm_bf_##n##_k16}
+    static const int tab[2][2][6] = {{VX_B6(kk), VX_B6(kx)}, {VX_B6(xk), VX_B6(xx)}};
+#undef VX_B6
     // A / B with stride 1 along K: 16-byte loads along it (4-byte aligned: any row stride); else along M / N
     const int k = tab[g.as[3] == 1 ? 0 : 1][g.bs[2] == 1 ? 0 : 1][cfg];
     const uint32_t tm = kBfRows[cfg], tn = kBfCols[cfg];
     // two buffers of a stage's terms (6 bytes an element) and a word; the K split: the waves' sums and 64 words
-    const size_t lds = cfg == BF_KS ? 8u * 4096u + 256u : (size_t)(tm + tn) * (cfg == BF_S2 ? 64u : 32u) * 12u + 16u;
+    const size_t lds = cfg >= BF_KS ? 8u * tm * tn * 4u + (tm + tn) * 4u
+                                    : (size_t)(tm + tn) * (cfg == BF_S2 ? 64u : 32u) * 12u + 16u;
     // a grid holds fewer than 2^32 threads: at most 2^21 tiles per launch
     const uint32_t sm = tm << 10, sn = tn << 11;
     for (uint64_t m = 0; m < g.M; m += sm)
@@ -476,7 +480,7 @@ static int run_gemm(vx_ctx ctx, vx_stream stream, const vx_mview* out, const vx_
     // 200 x 64, batch 40 10.3 / 14.1; but 1024 x 1024 x 64, batch 8 20.9 /
     // 16.7 and 3040 x 384 x 160 13.0 / 12.5).
     const bool shortk = p.K < 160u && am == 0 && bm != 2 && tiles(64, 64) <= 6ull * (uint64_t)ctx->num_cus;
-    if (cfg == BF_KS || !shortk) return launch_gemm_bf(ctx, stream, a, cfg, batch);
+    if (cfg >= BF_KS || !shortk) return launch_gemm_bf(ctx, stream, a, cfg, batch);
     const uint64_t tn = tiles(128, 128), tw = tiles(128, 256), ts = tiles(64, 64);
     // Tile shape. 128 x 256 tiles (two resident workgroups per CU) instead of
     // 128 x 128 (three) when they fill the last round of resident workgroups
