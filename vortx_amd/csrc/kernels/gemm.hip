@@ -177,8 +177,7 @@ __device__ __forceinline__ void vx_gemm_mfma(const vx_gemm_args& p) {
     // groups of 8 tile-rows so an XCD's resident tiles share A and B panels
     // in its L2.
     const uint32_t nt = p.tiles_m * p.tiles_n;
-    uint32_t bid = blockIdx.x;
-    if ((nt & 7u) == 0) bid = (bid & 7u) * (nt >> 3) + (bid >> 3);
+    const uint32_t bid = vx_xcd_order(blockIdx.x, nt);
     const uint32_t group = 8u * p.tiles_n;
     const uint32_t first_m = (bid / group) * 8u;
     const uint32_t gsize = min(p.tiles_m - first_m, 8u);

@@ -22,6 +22,7 @@
 
 #include "../vx_kargs.h"
 #include "vx_bf16.hpp"
+#include "vx_dpp.hpp"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -30,13 +31,6 @@ typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // Operand access: "x" is the non-K dimension (M for A, N for B).
 #define MODE_K 0  // stride 1 along K
 #define MODE_X 1  // any strides; best with stride 1 along x
-
-// Workgroup ids are dealt round robin to 8 XCDs: the id's place when each XCD
-// takes a contiguous run of tiles (any number of them: with runs only for
-// multiples of 8, 21 x 4588 x 1991 in 574 tiles took 35 us instead of 20.6).
-__device__ __forceinline__ uint32_t vx_xcd_order(uint32_t bid, uint32_t nt) {
-    return (bid & 7u) * (nt >> 3) + min(bid & 7u, nt & 7u) + (bid >> 3);
-}
 
 __device__ __forceinline__ void vx_epilogue(float* c, float acc, float alpha, float beta) {
     *c = beta == 0.f ? alpha * acc : alpha * acc + beta * *c;

@@ -135,3 +135,11 @@ __device__ __forceinline__ void vx_gather4(uint32_t v, uint32_t (&o)[4]) {
     o[2] = b;
     o[3] = b2;
 }
+
+// Workgroup ids are dealt round robin to 8 XCDs: the id's place when each XCD
+// takes a contiguous run of tiles (any number of them: with runs only for
+// multiples of 8, a GEMM of 21 x 4588 x 1991 in 574 tiles took 35 us instead of
+// 20.6).
+__device__ __forceinline__ uint32_t vx_xcd_order(uint32_t bid, uint32_t nt) {
+    return (bid & 7u) * (nt >> 3) + min(bid & 7u, nt & 7u) + (bid >> 3);
+}
