@@ -245,7 +245,7 @@ int vx_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y,
  * 1.6e-5 max|x_block|; products and block sums with the exactly decoded
  * weights are exact in int32 and the scaling is f32. Batch 1 reduces with
  * v_dot4_i32_i8, batches (B >= 2) on the int8 matrix cores. VX_GEMV_X_F32
- * keeps x in f32 instead (f32 FMA on the exactly decoded weights; slower);
+ * keeps x in f32 instead (on the exactly decoded weights; slower);
  * VX_GEMV_X_INT8 names the default split and may not be combined with it. */
 typedef enum vx_gemv_flags { VX_GEMV_X_INT8 = 1, VX_GEMV_X_F32 = 2 } vx_gemv_flags;
 /* With VX_GEMV_X_INT8, a batched shape whose split needs device memory
