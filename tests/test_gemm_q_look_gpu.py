@@ -1,0 +1,76 @@
+"""Products of a quantized W with many columns of x: outputs that the bf16 terms
+of x cannot form (infinities, sums beyond the largest float, x below what the
+terms hold) are formed from f32 products, at a bounded cost."""
+import pytest
+import torch
+
+import vortx_amd as vx
+from tests.helpers import note
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BLOCK = {vx.VX_Q4_0: (32, 18), vx.VX_Q8_0: (32, 34), vx.VX_Q4_K: (256, 144)}
+QTYPES = pytest.mark.parametrize("qtype", list(BLOCK), ids=["q4_0", "q8_0", "q4_k"])
+
+
+def _weights(qgemv, qtype, M, K, seed, zero=0):
+    """A quantized normal matrix (its first `zero` columns zeros), and its values."""
+    qk, bb = BLOCK[qtype]
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    v = torch.randn(M, K, device=DEV, generator=g) * K ** -0.5
+    v[:, :zero] = 0.0
+    w = vx.QWeight(torch.empty(M * (K // qk) * bb, dtype=torch.uint8, device=DEV), qtype, M, K)
+    qgemv.quantize(w, v)
+    wd = torch.empty(M, K, device=DEV)
+    qgemv.dequantize(wd, w)
+    return w, wd
+
+
+def _x(B, K, seed):
+    return torch.randn(B, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(seed))
+
+
+def _bound(x, wd, exact_x):
+    """|error|: a few f32 roundings per 32-block of the magnitudes added (at most
+    3 times the block's largest weight per element of x), and x to 2^-16."""
+    K = x.shape[1]
+    mag = 3.0 * wd.double().abs().view(-1, K // 32, 32).amax(-1).repeat_interleave(32, 1)
+    return ((K / 32 + 48) * 2.0 ** -24 + (0.0 if exact_x else 2.0 ** -16)) * (x.double().abs() @ mag.t())
+
+
+def _us(f):
+    f()
+    best = float("inf")
+    for _ in range(5):
+        t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        t0.record()
+        f()
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1) * 1e3)
+    return best
+
+
+@QTYPES
+@pytest.mark.parametrize("M,B", [(2000, 40), (2300, 1500)])
+def test_cost_of_non_finite_x(qgemv, qtype, M, B):
+    """A NaN or an infinity in every column: the outputs of the f32 products,
+    and a bounded time (measured 2 times a finite x's with NaNs, 4 to 7 times with
+    infinities; forming each output in one lane took 22 times and more)."""
+    K = 2048
+    note(f"gemm_q cost of non-finite {qtype} {M} B={B}")
+    w, wd = _weights(qgemv, qtype, M, K, 1)
+    x = _x(B, K, 2)
+    y = torch.empty(B, M, device=DEV)
+    call = lambda v: qgemv.dispatch(y.t(), w, v.t(), x_f32=True)  # noqa: E731
+    base = _us(lambda: call(x))
+    for bad in (float("nan"), float("inf")):
+        xb = x.clone()
+        xb[torch.arange(B), torch.arange(B) % K] = bad
+        us = _us(lambda: call(xb))
+        note(f"  {bad}: {us:.0f} us, {base:.0f} without")
+        want = xb.double() @ wd.double().t()
+        assert torch.equal(y.isnan(), want.isnan())
+        inf = want.isinf()
+        assert torch.equal(y[inf].double(), want[inf])
+        assert us < 12 * base + 50, f"{bad}: {us:.0f} us, {base:.0f} without"

@@ -170,29 +170,125 @@ __device__ __forceinline__ void vx_x8(const float* p, int64_t xs_k, float (&v)[8
     }
 }
 
-// A result that is not finite in the exact-x form is formed again the plain
-// way, one product at a time: the terms of an infinite x hold a NaN, where
-// the f32 products give an infinity.
-template <int QT>
-__device__ __forceinline__ float vx_gemm_q_redo(const vx_gemv_args& a, uint32_t row, uint32_t col) {
-    float s = 0.f;
-    for (uint32_t kb = 0; kb < a.K / 32u; ++kb) {
-        float o[32];
-        vx_decode32<QT>(a.w + (uint64_t)row * a.row_stride, kb, o);
-        const float* xp = a.x + (int64_t)col * a.xs_b + (int64_t)(32u * kb) * a.xs_k;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) s = __builtin_fmaf(o[i], xp[(int64_t)i * a.xs_k], s);
-    }
-    return s;
-}
-
-template <int QT, int NT>
-__device__ __forceinline__ void vx_gemm_q_store(const vx_gemv_args& a, uint32_t row, uint32_t col, float v) {
-    if (NT == 3 && !(__builtin_fabsf(v) < __builtin_inff())) v = vx_gemm_q_redo<QT>(a, row, col);
-    a.y[(int64_t)row * a.ys_m + (int64_t)col * a.ys_b] = v;
-}
-
 extern __shared__ __align__(16) uint8_t vx_gq_lds[];
+
+// Weights 8g..8g+7 of 32-block kb of a row as they are (load), and as floats.
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
+typedef uint16_t u16_a1 __attribute__((aligned(1)));
+template <int QT>
+struct vx_w8 {
+    uint32_t q0, q1, h, s1, s2, s3;
+    __device__ __forceinline__ void load(const uint8_t* row, uint32_t kb, uint32_t g) {
+        const uint8_t* p = row + (QT == VX_Q4_0 ? 18u * kb : QT == VX_Q8_0 ? 34u * kb : 144u * (kb >> 3));
+        const uint8_t* q = p + (QT == VX_Q4_0 ? 2u + 8u * (g & 1u) : QT == VX_Q8_0 ? 2u + 8u * g : 16u + 32u * ((kb & 7u) >> 1) + 8u * g);
+        q0 = *(const u32_a1*)q;
+        q1 = *(const u32_a1*)(q + 4);
+        if constexpr (QT == VX_Q4_K) {
+            h = *(const u32_a1*)p;
+            s1 = *(const u32_a1*)(p + 4);
+            s2 = *(const u32_a1*)(p + 8);
+            s3 = *(const u32_a1*)(p + 12);
+        } else {
+            h = *(const u16_a1*)p;
+        }
+    }
+    __device__ __forceinline__ void decode(uint32_t kb, uint32_t g, float (&o)[8]) const {
+        const float d = vx_f16_to_f32(h);
+        if constexpr (QT == VX_Q8_0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = d * (float)(int8_t)(((e < 4 ? q0 : q1) >> (8 * (e & 3))) & 0xFFu);
+        } else {
+            const uint32_t sh = 4u * (QT == VX_Q4_0 ? g >> 1 : kb & 1u);
+            uint32_t sc0, m0, sc1, m1;
+            if constexpr (QT == VX_Q4_K) vx_q4k_scales(s1, s2, s3, (kb & 7u) >> 1, sc0, m0, sc1, m1);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t n = ((e < 4 ? q0 : q1) >> (8u * (e & 3) + sh)) & 15u;
+                if constexpr (QT == VX_Q4_0) o[e] = (float)((int)n - 8) * d;
+                else o[e] = __fsub_rn(__fmul_rn(d * (float)((kb & 1u) ? sc1 : sc0), (float)n), vx_f16_to_f32(h >> 16) * (float)((kb & 1u) ? m1 : m0));
+            }
+        }
+    }
+};
+
+// A workgroup whose outputs hold one that is not finite looks at all of them
+// again (they are in y): the terms of an infinite x hold a NaN, where the f32
+// products give an infinity. Where the column of x holds a NaN, so does the
+// output; any other is formed again from f32 products, 16 x 16 CG outputs of a
+// wave on v_mfma_f32_16x16x4f32 (lane (n, g) of either operand holds elements
+// 8g..8g+7 of a block; U blocks requested ahead of their products).
+// Bound by its requests (16 rows of x and of W an instruction). Q4_0 2300 x 2048,
+// 1500 columns, three terms, us: 104; with a NaN in every column 198 (the look
+// alone), with an infinity in every one 643 (1210 with CG 1); one lane per output,
+// as before, 2275 and more.
+template <int QT, int NT, bool XV, uint32_t ROWS, uint32_t COLS, uint32_t NWV>
+__device__ __forceinline__ void vx_gemm_q_look(const vx_gemv_args& a, uint32_t row0, uint32_t col0) {
+    constexpr uint32_t CG = COLS >= 64u ? 4u : 1u, U = CG == 1u ? 4u : 2u;
+    const uint32_t t = threadIdx.x, lane = t & 63u, n = lane & 15u, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    uint32_t* mx = (uint32_t*)vx_gq_lds;  // [COLS]
+    __syncthreads();
+    for (uint32_t i = t; i < COLS; i += 64u * NWV) mx[i] = 0u;
+    __syncthreads();
+    vx_scan<XV, COLS>(a.x, a.xs_b, a.xs_k, col0, a.B, a.K, wave, NWV, lane, mx);
+    __syncthreads();
+    const uint32_t nblk = a.K / 32u;
+    for (uint32_t u = wave; u < ROWS / 16u * (COLS / (16u * CG)); u += NWV) {
+        const uint32_t r0 = row0 + u % (ROWS / 16u) * 16u, c0 = u / (ROWS / 16u) * (16u * CG);
+        if (r0 >= a.M || col0 + c0 >= a.B) continue;
+        float* y = a.y + (int64_t)(r0 + n) * a.ys_m + (int64_t)(col0 + c0 + 4u * g) * a.ys_b;  // columns 4g..4g+3 of each subtile
+        uint32_t again = 0u;
+#pragma unroll
+        for (uint32_t e = 0; e < 4u * CG; ++e) {
+            const uint32_t c = 16u * (e >> 2) + (e & 3u), cc = c0 + 4u * g + c;
+            if (r0 + n < a.M && col0 + cc < a.B && mx[cc] <= 0x7F800000u &&
+                !(__builtin_fabsf(y[(int64_t)c * a.ys_b]) < __builtin_inff()))
+                again |= 1u << e;
+        }
+        if (!__any(again != 0u)) continue;
+        const uint8_t* row = a.w + (uint64_t)min(r0 + n, a.M - 1u) * a.row_stride;
+        const float* xp[CG];
+#pragma unroll
+        for (uint32_t c = 0; c < CG; ++c)
+            xp[c] = a.x + (int64_t)min(col0 + c0 + 16u * c + n, a.B - 1u) * a.xs_b + (int64_t)(8u * g) * (XV ? 1 : a.xs_k);
+        f32x4 acc[CG];
+#pragma unroll
+        for (uint32_t c = 0; c < CG; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (uint32_t kb = 0; kb < nblk; kb += U) {
+            vx_w8<QT> w[U];
+            float xv[U][CG][8];
+#pragma unroll
+            for (uint32_t v = 0; v < U; ++v) {
+                const uint32_t k = min(kb + v, nblk - 1u);
+                w[v].load(row, k, g);
+#pragma unroll
+                for (uint32_t c = 0; c < CG; ++c) {
+                    const float* p = xp[c] + (int64_t)(32u * k) * (XV ? 1 : a.xs_k);
+                    if constexpr (XV) {
+                        *(f32x4*)&xv[v][c][0] = *(const f32x4*)p;
+                        *(f32x4*)&xv[v][c][4] = *(const f32x4*)(p + 4);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) xv[v][c][i] = p[(int64_t)i * a.xs_k];
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t v = 0; v < U; ++v) {
+                if (kb + v >= nblk) break;
+                float wv[8];
+                w[v].decode(kb + v, g, wv);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (uint32_t c = 0; c < CG; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[v][c][i], wv[i], acc[c], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < 4u * CG; ++e)
+            if (again >> e & 1u) y[(int64_t)(16u * (e >> 2) + (e & 3u)) * a.ys_b] = acc[e >> 2][e & 3u];
+    }
+}
 
 // K split over the waves of a workgroup: 16 WR rows x 16 CT columns per
 // workgroup, wave w takes the items w, w + NW, ... and reads its x itself.
@@ -292,6 +388,8 @@ __device__ __forceinline__ void vx_gemm_q_ks(const vx_gemv_args& a) {
     // red[wave][tile][e][lane]: the waves' sums in wave order
     float* red = (float*)vx_gq_lds;
     constexpr uint32_t PW = WR * CT * 256u;
+    uint32_t* word = (uint32_t*)(red + PW * NWV);  // whether an output needs a second look
+    if (t == 0u) *word = 0u;
 #pragma unroll
     for (int i = 0; i < WR; ++i)
 #pragma unroll
@@ -299,13 +397,20 @@ __device__ __forceinline__ void vx_gemm_q_ks(const vx_gemv_args& a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) red[wave * PW + (uint32_t)((i * CT + c) * 4 + e) * 64u + lane] = acc[i][c][e];
     __syncthreads();
+    bool look = false;
     for (uint32_t o = t; o < PW; o += 64u * NWV) {
         float s = red[o];
 #pragma unroll
         for (int k = 1; k < NWV; ++k) s += red[(uint32_t)k * PW + o];
         const uint32_t l = o & 63u, e = (o >> 6) & 3u, tile = o >> 8;
         const uint32_t row = row0 + 16u * (tile / CT) + (l & 15u), cc = col0 + 16u * (tile % CT) + 4u * (l >> 4) + e;
-        if (row < a.M && cc < a.B) vx_gemm_q_store<QT, NT>(a, row, cc, s);
+        if (row < a.M && cc < a.B) a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = s;
+        look = look || !(__builtin_fabsf(s) < __builtin_inff());
+    }
+    if constexpr (NT == 3) {
+        if (look) *word = 1u;
+        __syncthreads();
+        if (*word) vx_gemm_q_look<QT, NT, XV, 16u * WR, 16u * CT, NWV>(a, row0, col0);
     }
 }
 
@@ -351,6 +456,8 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
     uint8_t* W = (uint8_t*)(X + 2u * XB);           // [ROWS][IB]
     float* S = (float*)(W + ROWS * IB);             // OFF: [2 items][8 blocks][2 halves][COLS] sums of x
     uint32_t wlo = (64u * wm + n) * IB;             // this lane's row of row tile 0
+    uint32_t* word = (uint32_t*)(S + (OFF ? 32u * COLS : 0u));  // whether an output needs a second look
+    if (t == 0u) *word = 0u;
 
     f32x16 acc[2][2];
 #pragma unroll
@@ -624,7 +731,7 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
         offsets(nfull, nblk & 7u);
     }
     scale(1, 1, 1, 1);  // the last block's number is odd
-    bool fin = true;
+    bool look = false;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -633,19 +740,13 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
             for (int v = 0; v < 16; ++v) {
                 const uint32_t row = row0 + 64u * wm + 32u * i + n;
                 const uint32_t cc = col0 + 64u * wn + 32u * c + 8u * (v >> 2) + 4u * g + (v & 3);
-                if (row < a.M && cc < a.B) {
-                    a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = acc[i][c][v];
-                    fin = fin && __builtin_fabsf(acc[i][c][v]) < __builtin_inff();
-                }
+                if (row < a.M && cc < a.B) a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = acc[i][c][v];
+                look = look || !(__builtin_fabsf(acc[i][c][v]) < __builtin_inff());
             }
-    if (NT == 3 && !fin) {
-        for (uint32_t o = 0; o < 64u; ++o) {
-            const uint32_t row = row0 + 64u * wm + 32u * (o >> 5) + n;
-            const uint32_t cc = col0 + 64u * wn + 32u * ((o >> 4) & 1u) + 8u * ((o >> 2) & 3u) + 4u * g + (o & 3u);
-            if (row >= a.M || cc >= a.B) continue;
-            float* y = a.y + (int64_t)row * a.ys_m + (int64_t)cc * a.ys_b;
-            if (!(__builtin_fabsf(*y) < __builtin_inff())) *y = vx_gemm_q_redo<QT>(a, row, cc);
-        }
+    if constexpr (NT == 3) {
+        if (look) *word = 1u;
+        __syncthreads();
+        if (*word) vx_gemm_q_look<QT, NT, XV, ROWS, COLS, NWV>(a, row0, col0);
     }
 }
 

@@ -73,3 +73,22 @@ __device__ __forceinline__ void vx_split8_rne(const float (&v)[8], u32x4 (&t)[3]
             r[2 * i + 1] -= __uint_as_float(h & 0xFFFF0000u);
         }
 }
+
+// A second look at the T rows (or columns) x0.. of an operand, element (x, k) at
+// base[x sx + k sk]; those past X repeat the last. mx[x]: the bits of the largest
+// |element| (above 0x7F800000: it holds a NaN). Lanes follow K where that is the
+// dimension of stride 1 (KC), else x. All nw waves of the workgroup take part;
+// mx is in LDS, zeroed before.
+template <bool KC, uint32_t T>
+__device__ __forceinline__ void vx_scan(const float* base, int64_t sx, int64_t sk, uint32_t x0, uint32_t X, uint32_t K,
+                                        uint32_t wave, uint32_t nw, uint32_t lane, uint32_t* mx) {
+    constexpr uint32_t L = T < 64u ? T : 64u;  // lanes along x
+    for (uint32_t x = KC ? wave : lane % L; x < T; x += KC ? nw : L) {
+        const float* p = base + (int64_t)min(x0 + x, X - 1u) * sx;
+        uint32_t m = 0u;
+        const uint64_t k0 = KC ? lane : wave * (64u / L) + lane / L, step = KC ? 64u : nw * (64u / L);
+#pragma unroll 4
+        for (uint64_t k = k0; k < K; k += step) m = max(m, __float_as_uint(p[(int64_t)k * sk]) & 0x7FFFFFFFu);
+        atomicMax(&mx[x], m);
+    }
+}
