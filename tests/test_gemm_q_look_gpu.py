@@ -54,9 +54,9 @@ def _us(f):
 @QTYPES
 @pytest.mark.parametrize("M,B", [(2000, 40), (2300, 1500)])
 def test_cost_of_non_finite_x(qgemv, qtype, M, B):
-    """A NaN or an infinity in every column: the outputs of the f32 products,
-    and a bounded time (measured 2 times a finite x's with NaNs, 4 to 7 times with
-    infinities; forming each output in one lane took 22 times and more)."""
+    """A NaN or an infinity in every column, or only zeros: the outputs of the f32 products,
+    and a bounded time (measured 1.4 times an ordinary x's with NaNs or zeros, 3 to 6
+    times with infinities; forming each output in one lane took 22 times and more)."""
     K = 2048
     note(f"gemm_q cost of non-finite {qtype} {M} B={B}")
     w, wd = _weights(qgemv, qtype, M, K, 1)
@@ -64,8 +64,8 @@ def test_cost_of_non_finite_x(qgemv, qtype, M, B):
     y = torch.empty(B, M, device=DEV)
     call = lambda v: qgemv.dispatch(y.t(), w, v.t(), x_f32=True)  # noqa: E731
     base = _us(lambda: call(x))
-    for bad in (float("nan"), float("inf")):
-        xb = x.clone()
+    for bad in (float("nan"), float("inf"), 0.0):
+        xb = x.clone() if bad else torch.zeros_like(x)
         xb[torch.arange(B), torch.arange(B) % K] = bad
         us = _us(lambda: call(xb))
         note(f"  {bad}: {us:.0f} us, {base:.0f} without")
@@ -74,3 +74,26 @@ def test_cost_of_non_finite_x(qgemv, qtype, M, B):
         inf = want.isinf()
         assert torch.equal(y[inf].double(), want[inf])
         assert us < 12 * base + 50, f"{bad}: {us:.0f} us, {base:.0f} without"
+
+
+@QTYPES
+@pytest.mark.parametrize("M,B", [(300, 9), (2300, 1500)])
+@pytest.mark.parametrize("e", [-116, -122, -131])
+def test_small_x_keeps_its_bits(qgemv, qtype, M, B, e):
+    """x kept in f32 far below one (its third terms would fall below bf16's
+    smallest number, 2^-133): whole columns, and elements that are all that
+    counts beside larger ones whose weights are zeros."""
+    K = 512
+    note(f"gemm_q small x {qtype} {M} B={B} 2^{e}")
+    w, wd = _weights(qgemv, qtype, M, K, 3, zero=256)
+    x = _x(B, K, 4)
+    x[::2] = torch.ldexp(x[::2], torch.tensor(e, device=DEV))
+    x[1, 256:] = torch.ldexp(x[1, 256:], torch.tensor(e, device=DEV))
+    x[3, 300:] = 0.0
+    y, y2 = torch.empty(B, M, device=DEV), torch.empty(M, B, device=DEV)
+    qgemv.dispatch(y.t(), w, x.t(), x_f32=True)
+    qgemv.dispatch(y2, w, x.t().contiguous(), x_f32=True)
+    err = (y.double() - x.double() @ wd.double().t()).abs()
+    bound = _bound(x, wd, True) + K * 2.0 ** -149
+    assert (err <= bound).all(), f"{float((err / bound).max())} of the bound"
+    assert torch.equal(y, y2.t())

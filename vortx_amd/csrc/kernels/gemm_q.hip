@@ -211,39 +211,54 @@ struct vx_w8 {
     }
 };
 
-// A workgroup whose outputs hold one that is not finite looks at all of them
-// again (they are in y): the terms of an infinite x hold a NaN, where the f32
-// products give an infinity. Where the column of x holds a NaN, so does the
-// output; any other is formed again from f32 products, 16 x 16 CG outputs of a
-// wave on v_mfma_f32_16x16x4f32 (lane (n, g) of either operand holds elements
-// 8g..8g+7 of a block; U blocks requested ahead of their products).
+// Outputs that are not finite (the terms of an infinite x hold a NaN, where the
+// f32 products give an infinity) or below 2^-56 (the three terms of an x below
+// 2^-110 may miss bits, see vx_split8) are looked at again, in y, with the columns
+// of x that they came from. Where the column holds a NaN, so does the output. Any
+// other that is not finite, or whose column holds an x with missing bits, is
+// formed again from f32 products, 16 x 16 CG outputs of a wave on v_mfma_f32_16x16x4f32 (lane (n, g) of either operand holds elements
+// 8g..8g+7 of a block; U blocks requested ahead of their products). Above 2^-56
+// the missing bits, below 2^-133 of each x, are less than the roundings: with |w|
+// < 2^26 and K <= 2^28 they add up to 2^-79 at most, 2^-23 of the output.
 // Bound by its requests (16 rows of x and of W an instruction). Q4_0 2300 x 2048,
-// 1500 columns, three terms, us: 104; with a NaN in every column 198 (the look
-// alone), with an infinity in every one 643 (1210 with CG 1); one lane per output,
-// as before, 2275 and more.
+// 1500 columns, three terms, us: 106; with a NaN in every column 153 and with zeros
+// alone 141 (the look), with an infinity in every column 600 (each of these
+// outputs in one lane: 2275).
+__device__ __forceinline__ bool vx_gemm_q_odd(float y) {
+    const float v = __builtin_fabsf(y);
+    return !(v >= 0x1p-56f && v < __builtin_inff());
+}
+
+// odd[c]: whether column c of the workgroup holds such an output (in LDS, behind
+// what the look overwrites).
 template <int QT, int NT, bool XV, uint32_t ROWS, uint32_t COLS, uint32_t NWV>
-__device__ __forceinline__ void vx_gemm_q_look(const vx_gemv_args& a, uint32_t row0, uint32_t col0) {
+__device__ __forceinline__ void vx_gemm_q_look(const vx_gemv_args& a, uint32_t row0, uint32_t col0, const uint32_t* odd) {
     constexpr uint32_t CG = COLS >= 64u ? 4u : 1u, U = CG == 1u ? 4u : 2u;
     const uint32_t t = threadIdx.x, lane = t & 63u, n = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    uint32_t* mx = (uint32_t*)vx_gq_lds;  // [COLS]
+    uint32_t *mx = (uint32_t*)vx_gq_lds, *ls = mx + COLS;  // of each column
     __syncthreads();
-    for (uint32_t i = t; i < COLS; i += 64u * NWV) mx[i] = 0u;
+    if (!__any(odd[lane % COLS] != 0u || (COLS > 64u && odd[lane + 64u] != 0u))) return;  // (uniform over the workgroup)
+    for (uint32_t i = t; i < 2u * COLS; i += 64u * NWV) mx[i] = 0u;
     __syncthreads();
-    vx_scan<XV, COLS>(a.x, a.xs_b, a.xs_k, col0, a.B, a.K, wave, NWV, lane, mx);
+    vx_scan<XV, COLS>(a.x, a.xs_b, a.xs_k, col0, a.B, a.K, wave, NWV, lane, mx, ls,
+                      [&](uint32_t c) { return odd[c] != 0u; });
     __syncthreads();
     const uint32_t nblk = a.K / 32u;
     for (uint32_t u = wave; u < ROWS / 16u * (COLS / (16u * CG)); u += NWV) {
         const uint32_t r0 = row0 + u % (ROWS / 16u) * 16u, c0 = u / (ROWS / 16u) * (16u * CG);
         if (r0 >= a.M || col0 + c0 >= a.B) continue;
-        float* y = a.y + (int64_t)(r0 + n) * a.ys_m + (int64_t)(col0 + c0 + 4u * g) * a.ys_b;  // columns 4g..4g+3 of each subtile
+        float* y = a.y + (int64_t)min(r0 + n, a.M - 1u) * a.ys_m;
+        float v[4u * CG];  // columns 4g..4g+3 of each subtile (past the last: that one again)
+#pragma unroll
+        for (uint32_t e = 0; e < 4u * CG; ++e)
+            v[e] = y[(int64_t)min(col0 + c0 + 4u * g + 16u * (e >> 2) + (e & 3u), a.B - 1u) * a.ys_b];
         uint32_t again = 0u;
 #pragma unroll
         for (uint32_t e = 0; e < 4u * CG; ++e) {
-            const uint32_t c = 16u * (e >> 2) + (e & 3u), cc = c0 + 4u * g + c;
-            if (r0 + n < a.M && col0 + cc < a.B && mx[cc] <= 0x7F800000u &&
-                !(__builtin_fabsf(y[(int64_t)c * a.ys_b]) < __builtin_inff()))
-                again |= 1u << e;
+            const uint32_t cc = c0 + 4u * g + 16u * (e >> 2) + (e & 3u);
+            const bool in = (r0 + n < a.M) & (col0 + cc < a.B) & (mx[cc] <= 0x7F800000u);
+            again |= (uint32_t)(in & vx_gemm_q_odd(v[e]) & ((ls[cc] != 0u) | !(__builtin_fabsf(v[e]) < __builtin_inff()))) << e;
         }
         if (!__any(again != 0u)) continue;
         const uint8_t* row = a.w + (uint64_t)min(r0 + n, a.M - 1u) * a.row_stride;
@@ -273,6 +288,7 @@ __device__ __forceinline__ void vx_gemm_q_look(const vx_gemv_args& a, uint32_t r
                     }
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);  // (or the compiler moves each load to where it is used)
 #pragma unroll
             for (uint32_t v = 0; v < U; ++v) {
                 if (kb + v >= nblk) break;
@@ -286,7 +302,7 @@ __device__ __forceinline__ void vx_gemm_q_look(const vx_gemv_args& a, uint32_t r
         }
 #pragma unroll
         for (uint32_t e = 0; e < 4u * CG; ++e)
-            if (again >> e & 1u) y[(int64_t)(16u * (e >> 2) + (e & 3u)) * a.ys_b] = acc[e >> 2][e & 3u];
+            if (again >> e & 1u) y[(int64_t)(col0 + c0 + 4u * g + 16u * (e >> 2) + (e & 3u)) * a.ys_b] = acc[e >> 2][e & 3u];
     }
 }
 
@@ -388,8 +404,8 @@ __device__ __forceinline__ void vx_gemm_q_ks(const vx_gemv_args& a) {
     // red[wave][tile][e][lane]: the waves' sums in wave order
     float* red = (float*)vx_gq_lds;
     constexpr uint32_t PW = WR * CT * 256u;
-    uint32_t* word = (uint32_t*)(red + PW * NWV);  // whether an output needs a second look
-    if (t == 0u) *word = 0u;
+    uint32_t* odd = (uint32_t*)(red + PW * NWV);  // [16 CT], see vx_gemm_q_look
+    if (t < 16u * CT) odd[t] = 0u;
 #pragma unroll
     for (int i = 0; i < WR; ++i)
 #pragma unroll
@@ -397,7 +413,6 @@ __device__ __forceinline__ void vx_gemm_q_ks(const vx_gemv_args& a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) red[wave * PW + (uint32_t)((i * CT + c) * 4 + e) * 64u + lane] = acc[i][c][e];
     __syncthreads();
-    bool look = false;
     for (uint32_t o = t; o < PW; o += 64u * NWV) {
         float s = red[o];
 #pragma unroll
@@ -405,13 +420,9 @@ __device__ __forceinline__ void vx_gemm_q_ks(const vx_gemv_args& a) {
         const uint32_t l = o & 63u, e = (o >> 6) & 3u, tile = o >> 8;
         const uint32_t row = row0 + 16u * (tile / CT) + (l & 15u), cc = col0 + 16u * (tile % CT) + 4u * (l >> 4) + e;
         if (row < a.M && cc < a.B) a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = s;
-        look = look || !(__builtin_fabsf(s) < __builtin_inff());
+        if (NT == 3 && vx_gemm_q_odd(s)) odd[cc - col0] = 1u;
     }
-    if constexpr (NT == 3) {
-        if (look) *word = 1u;
-        __syncthreads();
-        if (*word) vx_gemm_q_look<QT, NT, XV, 16u * WR, 16u * CT, NWV>(a, row0, col0);
-    }
+    if constexpr (NT == 3) vx_gemm_q_look<QT, NT, XV, 16u * WR, 16u * CT, NWV>(a, row0, col0, odd);
 }
 
 // Tiles of 64 WM rows x 64 WN columns on v_mfma_f32_32x32x16_bf16; wave (wm,
@@ -456,8 +467,8 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
     uint8_t* W = (uint8_t*)(X + 2u * XB);           // [ROWS][IB]
     float* S = (float*)(W + ROWS * IB);             // OFF: [2 items][8 blocks][2 halves][COLS] sums of x
     uint32_t wlo = (64u * wm + n) * IB;             // this lane's row of row tile 0
-    uint32_t* word = (uint32_t*)(S + (OFF ? 32u * COLS : 0u));  // whether an output needs a second look
-    if (t == 0u) *word = 0u;
+    uint32_t* odd = (uint32_t*)(S + (OFF ? 32u * COLS : 0u));  // [COLS], see vx_gemm_q_look
+    if (t < COLS) odd[t] = 0u;
 
     f32x16 acc[2][2];
 #pragma unroll
@@ -731,7 +742,6 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
         offsets(nfull, nblk & 7u);
     }
     scale(1, 1, 1, 1);  // the last block's number is odd
-    bool look = false;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -741,13 +751,9 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
                 const uint32_t row = row0 + 64u * wm + 32u * i + n;
                 const uint32_t cc = col0 + 64u * wn + 32u * c + 8u * (v >> 2) + 4u * g + (v & 3);
                 if (row < a.M && cc < a.B) a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = acc[i][c][v];
-                look = look || !(__builtin_fabsf(acc[i][c][v]) < __builtin_inff());
+                if (NT == 3 && vx_gemm_q_odd(acc[i][c][v])) odd[cc - col0] = 1u;
             }
-    if constexpr (NT == 3) {
-        if (look) *word = 1u;
-        __syncthreads();
-        if (*word) vx_gemm_q_look<QT, NT, XV, ROWS, COLS, NWV>(a, row0, col0);
-    }
+    if constexpr (NT == 3) vx_gemm_q_look<QT, NT, XV, ROWS, COLS, NWV>(a, row0, col0, odd);
 }
 
 #define VX_GEMM_Q_KS(QT, QN, NT, WR, CT)                                                                  \

@@ -30,9 +30,10 @@ __device__ __forceinline__ uint32_t vx_pk_hi(uint32_t a, uint32_t b) {
 // v[0..8) as NT terms of packed bf16, largest first. The leading terms are
 // truncated (a rounded one could overflow to infinity for |v| near the
 // largest float; the remainder v - trunc(v) is exact either way). NT = 3: the
-// last term has at most 8 bits left, so the three add up to v exactly (down
-// to bf16's smallest subnormal, 2^-133). NT = 2: the last term is rounded,
-// error <= 2^-16 |v|. An infinity gives {inf, NaN, ..}, a NaN {NaN, ..}.
+// last term has at most 8 bits left, so the three add up to v exactly, except
+// for bits of v below 2^-133, bf16's smallest number (there are any only where
+// |v| < 2^-110). NT = 2: the last term is rounded, error <= 2^-16 |v|. An infinity
+// gives {inf, NaN, ..}, a NaN {NaN, ..}.
 template <int NT>
 __device__ __forceinline__ void vx_split8(const float (&v)[8], u32x4 (&t)[NT]) {
     float r[8];
@@ -74,21 +75,47 @@ __device__ __forceinline__ void vx_split8_rne(const float (&v)[8], u32x4 (&t)[3]
         }
 }
 
-// A second look at the T rows (or columns) x0.. of an operand, element (x, k) at
-// base[x sx + k sk]; those past X repeat the last. mx[x]: the bits of the largest
-// |element| (above 0x7F800000: it holds a NaN). Lanes follow K where that is the
-// dimension of stride 1 (KC), else x. All nw waves of the workgroup take part;
-// mx is in LDS, zeroed before.
-template <bool KC, uint32_t T>
+// A second look at those of the T rows (or columns) x0.. of an operand for which
+// want(x) holds, element (x, k) at base[x sx + k sk]; those past X repeat the
+// last. mx[x]: the bits of the largest |element| (above 0x7F800000: it holds a
+// NaN); ls[x]: whether three bf16 terms miss bits of an element (below 2^-110 and
+// no multiple of 2^-133, which adding 1.5 x 2^-110 rounds it to). Lanes follow K
+// where that is the dimension of stride 1 (KC), else x. All nw waves of the
+// workgroup take part; mx and ls are in LDS, zeroed before.
+template <bool KC, uint32_t T, class Want>
 __device__ __forceinline__ void vx_scan(const float* base, int64_t sx, int64_t sk, uint32_t x0, uint32_t X, uint32_t K,
-                                        uint32_t wave, uint32_t nw, uint32_t lane, uint32_t* mx) {
+                                        uint32_t wave, uint32_t nw, uint32_t lane, uint32_t* mx, uint32_t* ls,
+                                        Want want) {
     constexpr uint32_t L = T < 64u ? T : 64u;  // lanes along x
     for (uint32_t x = KC ? wave : lane % L; x < T; x += KC ? nw : L) {
+        if (!want(x)) continue;
         const float* p = base + (int64_t)min(x0 + x, X - 1u) * sx;
-        uint32_t m = 0u;
-        const uint64_t k0 = KC ? lane : wave * (64u / L) + lane / L, step = KC ? 64u : nw * (64u / L);
-#pragma unroll 4
-        for (uint64_t k = k0; k < K; k += step) m = max(m, __float_as_uint(p[(int64_t)k * sk]) & 0x7FFFFFFFu);
-        atomicMax(&mx[x], m);
+        uint32_t m = 0u, l = 0u;
+        auto take = [&](float v) {
+            const uint32_t u = __float_as_uint(v) & 0x7FFFFFFFu;
+            m = max(m, u);
+            l |= (uint32_t)(u < 0x08800000u /* 2^-110 */) & (uint32_t)((v + 0x1.8p-110f) - 0x1.8p-110f != v);
+        };
+        // 16 loads in flight
+        const uint32_t k0 = KC ? lane : wave * (64u / L) + lane / L, step = KC ? 64u : nw * (64u / L);
+        const int64_t ks = KC ? 1 : sk;
+        const float* q = p + (int64_t)k0 * ks;
+        uint64_t k = 0;
+        for (; k + 16u * step <= K; k += 16u * step, q += (int64_t)(16u * step) * ks) {
+            float v[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v[j] = q[(int64_t)j * (KC ? 64 : (int64_t)step * sk)];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) take(v[j]);
+        }
+        for (k += k0; k < K; k += step) take(p[(int64_t)k * ks]);
+        if constexpr (KC) {
+#pragma unroll
+            for (int o = 32; o; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+            if (lane == 0u) mx[x] = m;  // (no other wave has x)
+        } else {
+            atomicMax(&mx[x], m);
+        }
+        if (l) ls[x] = 1u;
     }
 }

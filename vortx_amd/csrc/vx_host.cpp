@@ -912,11 +912,11 @@ static int launch_gemm_q(vx_ctx ctx, vx_stream stream, const Canon& cy, const vx
     const int k = tab[q_index(w->qtype)][nt - 2][cfg][a.x_vec ? 0 : 1];
     const uint32_t rows = kGemmQRows[cfg], cols = kGemmQCols[cfg];
     const uint32_t nrow = (uint32_t)(((uint64_t)a.M + rows - 1u) / rows);
-    size_t lds;  // the waves' partial sums, or x (two buffers), W's rows of an item and the sums of x; a word
+    size_t lds;  // the waves' partial sums, or x (two buffers), W's rows of an item and the sums of x; a word per column
     if (cfg < 3) lds = (size_t)8u * rows * cols * 4u;
     else lds = (size_t)2u * 8u * (uint32_t)nt * 1024u + rows * (w->qtype == VX_Q8_0 ? 272u : 144u) +
                (w->qtype == VX_Q8_0 ? 0u : 2u * 8u * 2u * cols * 4u);
-    lds += 16u;
+    lds += cols * 4u;
     // a grid holds fewer than 2^32 threads: columns in slices of at most 2^22 workgroups
     const uint32_t slice = std::max(1u, (1u << 22) / nrow);
     for (uint64_t b0 = 0; b0 < B; b0 += (uint64_t)slice * cols) {
