@@ -228,10 +228,10 @@ int vx_gemm_f32_route(const vx_mview* out, const vx_cview* lhs,
  * is kept in f32; two, |error| <= 2^-16 |x| per element (closer than the int8
  * split), with a workspace. Products with the whole-number weights are exact,
  * sums and scaling f32. A non-finite x reaches its own column only, as on the
- * other routes; with three terms its outputs are formed from f32 products (a
+ * other routes; outputs that are not finite are formed from f32 products (a
  * call with an infinity in every column takes 3 to 6 times as long, with a NaN
- * in every column or with zeros alone 1.4 times), and so are the smallest outputs of a column that holds
- * an x below 2^-110, of which three terms may miss bits.
+ * in every column or with x in f32 and zeros alone 1.4 times), and so are, with x in f32, the smallest
+ * outputs of a column that holds an x below 2^-110, of which three terms may miss bits.
  * Empty shapes: K = 0 writes y = 0 (as vx_gemm_f32 with K = 0); M = 0 or
  * B = 0 returns VX_OK and launches nothing. The same holds for _ex, _ws
  * and _noalloc; vx_gemv_q_xq also returns VX_OK for M = 0 or B = 0 but

@@ -97,3 +97,20 @@ def test_small_x_keeps_its_bits(qgemv, qtype, M, B, e):
     bound = _bound(x, wd, True) + K * 2.0 ** -149
     assert (err <= bound).all(), f"{float((err / bound).max())} of the bound"
     assert torch.equal(y, y2.t())
+
+
+@QTYPES
+@pytest.mark.parametrize("M,B", [(300, 40), (2300, 1500)])
+def test_large_x_with_a_workspace(qgemv, qtype, M, B):
+    """x around 1e37 with a workspace: a block's whole-number sum (up to 32 x 127
+    times x) is beyond the largest float, the result is not."""
+    K = 512
+    note(f"gemm_q large x {qtype} {M} B={B}")
+    w, wd = _weights(qgemv, qtype, M, K, 5)
+    x = _x(B, K, 6).clamp_(-3, 3)
+    x[::2] *= 1e37
+    y = torch.empty(B, M, device=DEV)
+    qgemv.dispatch(y.t(), w, x.t(), workspace=vx.QuantGemv.workspace(w, B))
+    err = (y.double() - x.double() @ wd.double().t()).abs()
+    bound = _bound(x, wd, False)
+    assert (err <= bound).all(), f"{float((err / bound).max())} of the bound"

@@ -212,8 +212,9 @@ struct vx_w8 {
 };
 
 // Outputs that are not finite (the terms of an infinite x hold a NaN, where the
-// f32 products give an infinity) or below 2^-56 (the three terms of an x below
-// 2^-110 may miss bits, see vx_split8) are looked at again, in y, with the columns
+// f32 products give an infinity; a block's sum of whole numbers times x may pass
+// the largest float before the scale brings it back) or, with x exact, below 2^-56
+// (three terms of an x below 2^-110 may miss bits, see vx_split8) are looked at again, in y, with the columns
 // of x that they came from. Where the column holds a NaN, so does the output. Any
 // other that is not finite, or whose column holds an x with missing bits, is
 // formed again from f32 products, 16 x 16 CG outputs of a wave on v_mfma_f32_16x16x4f32 (lane (n, g) of either operand holds elements
@@ -224,9 +225,10 @@ struct vx_w8 {
 // 1500 columns, three terms, us: 106; with a NaN in every column 153 and with zeros
 // alone 141 (the look), with an infinity in every column 600 (each of these
 // outputs in one lane: 2275).
+template <int NT>
 __device__ __forceinline__ bool vx_gemm_q_odd(float y) {
     const float v = __builtin_fabsf(y);
-    return !(v >= 0x1p-56f && v < __builtin_inff());
+    return !((NT == 2 || v >= 0x1p-56f) && v < __builtin_inff());
 }
 
 // odd[c]: whether column c of the workgroup holds such an output (in LDS, behind
@@ -258,7 +260,7 @@ __device__ __forceinline__ void vx_gemm_q_look(const vx_gemv_args& a, uint32_t r
         for (uint32_t e = 0; e < 4u * CG; ++e) {
             const uint32_t cc = c0 + 4u * g + 16u * (e >> 2) + (e & 3u);
             const bool in = (r0 + n < a.M) & (col0 + cc < a.B) & (mx[cc] <= 0x7F800000u);
-            again |= (uint32_t)(in & vx_gemm_q_odd(v[e]) & ((ls[cc] != 0u) | !(__builtin_fabsf(v[e]) < __builtin_inff()))) << e;
+            again |= (uint32_t)(in & vx_gemm_q_odd<NT>(v[e]) & ((ls[cc] != 0u) | !(__builtin_fabsf(v[e]) < __builtin_inff()))) << e;
         }
         if (!__any(again != 0u)) continue;
         const uint8_t* row = a.w + (uint64_t)min(r0 + n, a.M - 1u) * a.row_stride;
@@ -420,9 +422,9 @@ __device__ __forceinline__ void vx_gemm_q_ks(const vx_gemv_args& a) {
         const uint32_t l = o & 63u, e = (o >> 6) & 3u, tile = o >> 8;
         const uint32_t row = row0 + 16u * (tile / CT) + (l & 15u), cc = col0 + 16u * (tile % CT) + 4u * (l >> 4) + e;
         if (row < a.M && cc < a.B) a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = s;
-        if (NT == 3 && vx_gemm_q_odd(s)) odd[cc - col0] = 1u;
+        if (vx_gemm_q_odd<NT>(s)) odd[cc - col0] = 1u;
     }
-    if constexpr (NT == 3) vx_gemm_q_look<QT, NT, XV, 16u * WR, 16u * CT, NWV>(a, row0, col0, odd);
+    vx_gemm_q_look<QT, NT, XV, 16u * WR, 16u * CT, NWV>(a, row0, col0, odd);
 }
 
 // Tiles of 64 WM rows x 64 WN columns on v_mfma_f32_32x32x16_bf16; wave (wm,
@@ -742,6 +744,17 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
         offsets(nfull, nblk & 7u);
     }
     scale(1, 1, 1, 1);  // the last block's number is odd
+    float f = 0.f, lo = 1.f;  // f: a NaN when an output is not finite
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                f = __builtin_fmaf(acc[i][c][v], 0.f, f);
+                lo = fminf(lo, __builtin_fabsf(acc[i][c][v]));
+            }
+    const bool look = f != 0.f || vx_gemm_q_odd<NT>(lo);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -751,9 +764,17 @@ __device__ __forceinline__ void vx_gemm_q_tile(const vx_gemv_args& a) {
                 const uint32_t row = row0 + 64u * wm + 32u * i + n;
                 const uint32_t cc = col0 + 64u * wn + 32u * c + 8u * (v >> 2) + 4u * g + (v & 3);
                 if (row < a.M && cc < a.B) a.y[(int64_t)row * a.ys_m + (int64_t)cc * a.ys_b] = acc[i][c][v];
-                if (NT == 3 && vx_gemm_q_odd(acc[i][c][v])) odd[cc - col0] = 1u;
             }
-    if constexpr (NT == 3) vx_gemm_q_look<QT, NT, XV, ROWS, COLS, NWV>(a, row0, col0, odd);
+    if (look) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (vx_gemm_q_odd<NT>(acc[i][c][v])) odd[64u * wn + 32u * c + 8u * (v >> 2) + 4u * g + (v & 3)] = 1u;
+    }
+    vx_gemm_q_look<QT, NT, XV, ROWS, COLS, NWV>(a, row0, col0, odd);
 }
 
 #define VX_GEMM_Q_KS(QT, QN, NT, WR, CT)                                                                  \
