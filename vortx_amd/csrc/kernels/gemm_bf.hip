@@ -48,7 +48,6 @@ struct vx_slab {
     static_assert(P * NTH == T * KG, "whole pieces");
     float r[D][P][8];  // D stages in flight
     const float* p[P];
-    float mx[P];  // largest |element| seen
 
     static __device__ __forceinline__ uint32_t px(int u) {
         const uint32_t i = threadIdx.x % NTH + (uint32_t)(NTH * u);
@@ -63,7 +62,6 @@ struct vx_slab {
         for (int u = 0; u < P; ++u) {
             const uint32_t x = min(x0 + px(u), X - 1u);
             p[u] = MODE == MODE_K ? base + (int64_t)x * sx + 8u * pk(u) : base + (int64_t)x * sx;
-            mx[u] = 0.f;
         }
     }
     // a stage inside K
@@ -92,12 +90,9 @@ struct vx_slab {
     // terms of piece u to LDS: [k16][x / 32][term][64 lanes], lane (n, g) of
     // an MFMA operand (row n, k 8g..8g+7) at g 32 + (n ^ 4 kg), kg = 2 k16 + g:
     // the xor spreads the pieces that 8 consecutive lanes store over the banks
-    __device__ __forceinline__ void store(int d, int u, u32x4* S) {
+    __device__ __forceinline__ void store(int d, int u, u32x4* S, uint32_t& lost) {
         u32x4 t[3];
-        vx_split8_rne(r[d][u], t);
-#pragma unroll
-        for (int j = 0; j < 8; j += 2)
-            mx[u] = fmaxf(fmaxf(__builtin_fabsf(r[d][u][j]), __builtin_fabsf(r[d][u][j + 1])), mx[u]);
+        vx_split8_rne(r[d][u], t, lost);
         const uint32_t x = px(u), kg = pk(u);
         u32x4* o = S + (((kg >> 1) * (T / 32) + (x >> 5)) * 3u) * 64u + (kg & 1u) * 32u + ((x & 31u) ^ (4u * kg));
 #pragma unroll
@@ -105,10 +100,23 @@ struct vx_slab {
     }
 };
 
-// Element (row, col) the plain way: an output that is not finite (the terms of
-// an infinity hold a NaN), or whose row of A or column of B holds nothing
-// above 2^-109 (its third terms fall below bf16's subnormals), or whose
-// products fall below 2^-80 (so would some of their parts).
+// Outputs of a tile that lost bits of an operand (vx_split8_rne), or that holds
+// an output for which odd() is true, are looked at again. The tile's rows of A
+// and columns of B are scanned (vx_scan), and an output is formed the plain way
+//   where it is not finite: the terms of an infinity hold a NaN;
+//   where it is below 2^-120: its six sums would be rounded to 2^-149 each;
+//   where an element of its row or column misses bits, up to 2^-134 each, and
+//   they may count: K 2^-134 max|b| + K 2^-134 max|a| against 2^-24 of it.
+// (The matrix cores keep subnormal operands, products and sums.)
+__device__ __forceinline__ bool vx_gemm_bf_odd(float s) {
+    const float v = __builtin_fabsf(s);
+    return !(v < __builtin_inff()) || (v < 0x1p-120f && v > 0.f);
+}
+// ra, cb: the bits of the largest |a| of the row and |b| of the column
+__device__ __forceinline__ bool vx_gemm_bf_again(float s, uint32_t K, uint32_t ra, bool rlost, uint32_t cb, bool clost) {
+    const float big = fmaxf(rlost ? __uint_as_float(cb) : 0.f, clost ? __uint_as_float(ra) : 0.f);
+    return vx_gemm_bf_odd(s) || ((rlost || clost) && !(__builtin_fabsf(s) >= (float)K * 0x1p-109f * big));
+}
 __device__ __forceinline__ float vx_gemm_bf_redo(const vx_gemm_args& p, const float* a, const float* b) {
     float s = 0.f;
     for (uint32_t k = 0; k < p.K; ++k) s = __builtin_fmaf(a[(int64_t)k * p.as[3]], b[(int64_t)k * p.bs[2]], s);
@@ -167,6 +175,7 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
     a.init(A, p.as[2], m0, p.M);
     b.init(B, p.bs[3], n0, p.N);
 
+    uint32_t lost = 0u;  // see vx_split8_rne
     const uint32_t nkf = p.K / BK;
     // accumulator q: half h of the stage in buffer buf
     auto mult = [&](uint32_t buf, int q, uint32_t h) {
@@ -205,11 +214,11 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
     auto store = [&](int d, uint32_t buf) {
         if (!DUTY || !dutyb) {
 #pragma unroll
-            for (int u = 0; u < PA; ++u) a.store(d, u, SAp + buf * SA);
+            for (int u = 0; u < PA; ++u) a.store(d, u, SAp + buf * SA, lost);
         }
         if (!DUTY || dutyb) {
 #pragma unroll
-            for (int u = 0; u < PB; ++u) b.store(d, u, SBp + buf * SB);
+            for (int u = 0; u < PB; ++u) b.store(d, u, SBp + buf * SB, lost);
         }
     };
     // stage st from its buffer; stage st + 1 is converted to the other one
@@ -225,10 +234,10 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
                 for (int u = 0; u < PA + PB; ++u) {
                     if (u * (NA * ST) / (PA + PB) != q) continue;
                     if (u < PA) {
-                        a.store(d, u, SAp + (buf ^ 1u) * SA);
+                        a.store(d, u, SAp + (buf ^ 1u) * SA, lost);
                         a.load(d, u, p.as[3], k2);
                     } else {
-                        b.store(d, u - PA, SBp + (buf ^ 1u) * SB);
+                        b.store(d, u - PA, SBp + (buf ^ 1u) * SB, lost);
                         b.load(d, u - PA, p.bs[2], k2);
                     }
                 }
@@ -279,15 +288,9 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
         for (int q = 0; q < NA * ST; ++q) mult(0u, q % NA, HS == 1 ? (uint32_t)q : 2u * (uint32_t)q + wh);
         __syncthreads();
     }
-    // Even + odd, to acc[0] (HS 2: of the even waves). Beside it one word says
-    // whether a thread saw only small elements in a piece (8 elements of a row
-    // or column per stage) with any: some output may then need a closer look.
+    // Even + odd, to acc[0] (HS 2: of the even waves). Beside it a word: whether
+    // the tile needs a closer look.
     uint32_t* word = (uint32_t*)(SBp + 2u * SB);
-    bool small = false;
-#pragma unroll
-    for (int u = 0; u < PA; ++u) small |= a.mx[u] < 0x1p-40f && a.mx[u] > 0.f;
-#pragma unroll
-    for (int u = 0; u < PB; ++u) small |= b.mx[u] < 0x1p-40f && b.mx[u] > 0.f;
     if (threadIdx.x == 0u) *word = 0u;
     float* red = (float*)vx_bf_lds + wave % (WM * WN) * (MI * NJ * 1024u) + lane;
     if (HS == 2 && wh) {
@@ -299,8 +302,12 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
                 for (int v = 0; v < 16; ++v) red[((i * NJ + j) * 16 + v) * 64] = acc[0][i][j][v];
     }
     __syncthreads();
-    if (small) *word = 1u;
+    if ((lost & 0xFFFFu) != 0u) *word = 1u;
     if (!wh) {
+        // f: a NaN when an output is not finite; lo: twice the bits of the
+        // smallest |output| above 0, less one
+        float f = 0.f;
+        uint32_t lo = ~0u;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -310,62 +317,51 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
 #pragma unroll
                     for (int v = 0; v < 16; ++v) acc[0][i][j][v] += red[((i * NJ + j) * 16 + v) * 64];
                 }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    f = __builtin_fmaf(acc[0][i][j][v], 0.f, f);
+                    lo = min(lo, (__float_as_uint(acc[0][i][j][v]) << 1) - 1u);
+                }
             }
+        if (f != 0.f || lo < (0x03800000u << 1) - 1u /* 2^-120 */) *word = 1u;
     }
     __syncthreads();
     const bool look = *word != 0u;
     const uint32_t rt0 = wm * (32u * MI) + 4u * g, ct0 = wn * (32u * NJ) + n;
     float* c0 = C + (int64_t)(m0 + rt0) * p.cs[2] + (int64_t)(n0 + ct0) * p.cs[3];
-    uint64_t again = 0;  // outputs to form the plain way
-    static_assert(MI * NJ * 16 <= 64, "one bit per output of a lane");
-    if (!wh) {
-        float f = 0.f;  // NaN when an output is not finite
+    if (!look && !wh && m0 + TM <= p.M && n0 + TN <= p.N) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) f = __builtin_fmaf(acc[0][i][j][v], 0.f, f);
-        if (!__any(f != 0.f || look) && m0 + TM <= p.M && n0 + TN <= p.N) {
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int i = 0; i < MI; ++i)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        vx_epilogue(c0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * p.cs[2] + (int64_t)(32 * j) * p.cs[3],
-                                    acc[0][i][j][v], p.alpha, p.beta);
-            return;  // (look is clear: no barrier follows for the workgroup)
-        }
+                for (int v = 0; v < 16; ++v)
+                    vx_epilogue(c0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * p.cs[2] + (int64_t)(32 * j) * p.cs[3],
+                                acc[0][i][j][v], p.alpha, p.beta);
+        return;
     }
-    uint32_t* mx = (uint32_t*)vx_bf_lds;  // [TM + TN] the largest |element| of each row of A and column of B
+    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + TM + TN;  // of each row of A and column of B, see vx_scan
     if (look) {
-        for (uint32_t i = threadIdx.x; i < TM + TN; i += NTH) mx[i] = 0u;
+        for (uint32_t i = threadIdx.x; i < 2u * (TM + TN); i += NTH) mx[i] = 0u;
         __syncthreads();
-        if (!DUTY || !dutyb) {
-#pragma unroll
-            for (int u = 0; u < PA; ++u) atomicMax(&mx[a.px(u)], __float_as_uint(a.mx[u]));
-        }
-        if (!DUTY || dutyb) {
-#pragma unroll
-            for (int u = 0; u < PB; ++u) atomicMax(&mx[TM + b.px(u)], __float_as_uint(b.mx[u]));
-        }
+        auto all = [](uint32_t) { return true; };
+        vx_scan<AM == MODE_K, TM>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NTH / 64, lane, mx, ls, all);
+        vx_scan<BM == MODE_K, TN>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NTH / 64, lane, mx + TM, ls + TM, all);
         __syncthreads();
     }
     if (wh) return;
+    uint64_t again = 0;  // outputs to form the plain way
+    static_assert(MI * NJ * 16 <= 64, "one bit per output of a lane");
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const uint32_t ct = ct0 + 32u * j;
-        const float cm = look ? __uint_as_float(mx[TM + ct]) : 1.f;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const uint32_t rt = rt0 + 32u * i + 8u * (v >> 2) + (v & 3);
-                const float rm = look ? __uint_as_float(mx[rt]) : 1.f;
                 if (m0 + rt < p.M && n0 + ct < p.N) {
-                    const bool tiny = (rm * cm < 0x1p-80f || fminf(rm, cm) < 0x1p-109f) && rm > 0.f && cm > 0.f;
-                    if (__builtin_fabsf(acc[0][i][j][v]) < __builtin_inff() && !tiny)
+                    if (!look || !vx_gemm_bf_again(acc[0][i][j][v], p.K, mx[rt], ls[rt] != 0u, mx[TM + ct], ls[TM + ct] != 0u))
                         vx_epilogue(c0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * p.cs[2] + (int64_t)(32 * j) * p.cs[3],
                                     acc[0][i][j][v], p.alpha, p.beta);
                     else
@@ -435,18 +431,13 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
     f32x16 acc[2];
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.f;
-    float ma = 0.f, mb = 0.f;  // the largest |element| seen
+    uint32_t lost = 0u;  // see vx_split8_rne
     auto mult = [&](const vx_chunk<AM>& a, const vx_chunk<BM>& b) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             u32x4 ta[3], tb[3];
-            vx_split8_rne(a.r[h], ta);
-            vx_split8_rne(b.r[h], tb);
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                ma = fmaxf(fmaxf(__builtin_fabsf(a.r[h][j]), __builtin_fabsf(a.r[h][j + 1])), ma);
-                mb = fmaxf(fmaxf(__builtin_fabsf(b.r[h][j]), __builtin_fabsf(b.r[h][j + 1])), mb);
-            }
+            vx_split8_rne(a.r[h], ta, lost);
+            vx_split8_rne(b.r[h], tb, lost);
             constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};  // smallest products first
 #pragma unroll
             for (int e = 0; e < 6; ++e)
@@ -485,29 +476,40 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
         b.load_tail(pb, p.bs[2], nck * 32u, g, p.K);
         mult(a, b);
     }
-    // red[wave][v][lane], and the largest elements of the tile's rows of A and columns of B
+    // red[wave][v][lane], and whether the tile needs a closer look
     float* red = (float*)vx_bf_lds;
-    uint32_t* mx = (uint32_t*)(red + NWV * 1024u);
-    if (t < 64u) mx[t] = 0u;
+    uint32_t* word = (uint32_t*)(red + NWV * 1024u);
+    if (t == 0u) *word = 0u;
 #pragma unroll
     for (int v = 0; v < 16; ++v) red[wave * 1024u + (uint32_t)v * 64u + lane] = acc[0][v] + acc[1][v];
     __syncthreads();
-    atomicMax(&mx[n], __float_as_uint(ma));
-    atomicMax(&mx[32u + n], __float_as_uint(mb));
+    float s[2];
+#pragma unroll
+    for (uint32_t u = 0; u < 2u; ++u) {
+        s[u] = red[t + 512u * u];
+#pragma unroll
+        for (uint32_t w = 1; w < NWV; ++w) s[u] += red[w * 1024u + t + 512u * u];
+    }
+    if ((lost & 0xFFFFu) != 0u || vx_gemm_bf_odd(s[0]) || vx_gemm_bf_odd(s[1])) *word = 1u;
     __syncthreads();
+    const bool look = *word != 0u;
+    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + 64;  // of each row of A and column of B, see vx_scan
+    if (look) {
+        if (t < 128u) mx[t] = 0u;
+        __syncthreads();
+        auto all = [](uint32_t) { return true; };
+        vx_scan<AM == MODE_K, 32>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NWV, lane, mx, ls, all);
+        vx_scan<BM == MODE_K, 32>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 32, ls + 32, all);
+        __syncthreads();
+    }
 #pragma unroll
-    for (uint32_t o = t; o < 1024u; o += 64u * NWV) {
-        float s = red[o];
-#pragma unroll
-        for (uint32_t w = 1; w < NWV; ++w) s += red[w * 1024u + o];
-        const uint32_t l = o & 63u, v = o >> 6, rt = 8u * (v >> 2) + 4u * (l >> 5) + (v & 3u), ct = l & 31u;
+    for (uint32_t u = 0; u < 2u; ++u) {
+        const uint32_t o = t + 512u * u, l = o & 63u, v = o >> 6, rt = 8u * (v >> 2) + 4u * (l >> 5) + (v & 3u), ct = l & 31u;
         const uint32_t row = m0 + rt, col = n0 + ct;
         if (row >= p.M || col >= p.N) continue;
-        const float rm = __uint_as_float(mx[rt]), cm = __uint_as_float(mx[32u + ct]);
-        const bool tiny = (rm * cm < 0x1p-80f || fminf(rm, cm) < 0x1p-109f) && rm > 0.f && cm > 0.f;
-        if (!(__builtin_fabsf(s) < __builtin_inff()) || tiny)
-            s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
-        vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+        if (look && vx_gemm_bf_again(s[u], p.K, mx[rt], ls[rt] != 0u, mx[32u + ct], ls[32u + ct] != 0u))
+            s[u] = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
+        vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s[u], p.alpha, p.beta);
     }
 }
 
@@ -563,16 +565,11 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
     const float* pb = B + (int64_t)min(n0 + n, p.N - 1u) * p.bs[3];
 
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // even and odd chunks
-    float ma = 0.f, mb = 0.f;  // the largest |element| seen
+    uint32_t lost = 0u;  // see vx_split8_rne
     auto mult = [&](const vx_strip<AM>& a, const vx_strip<BM>& b, int par) {
         u32x4 ta[3], tb[3];
-        vx_split8_rne(a.r, ta);
-        vx_split8_rne(b.r, tb);
-#pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-            ma = fmaxf(fmaxf(__builtin_fabsf(a.r[j]), __builtin_fabsf(a.r[j + 1])), ma);
-            mb = fmaxf(fmaxf(__builtin_fabsf(b.r[j]), __builtin_fabsf(b.r[j + 1])), mb);
-        }
+        vx_split8_rne(a.r, ta, lost);
+        vx_split8_rne(b.r, tb, lost);
         constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};  // smallest products first
 #pragma unroll
         for (int e = 0; e < 6; ++e)
@@ -608,26 +605,33 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
         b.load_tail(pb, p.bs[2], nck * 32u, g, p.K);
         mult(a, b, 1);
     }
-    // red[wave][v][lane], and the largest elements of the tile's rows of A and columns of B
+    // red[wave][v][lane], and whether the tile needs a closer look
     float* red = (float*)vx_bf_lds;
-    uint32_t* mx = (uint32_t*)(red + NWV * 256u);
-    if (t < 32u) mx[t] = 0u;
+    uint32_t* word = (uint32_t*)(red + NWV * 256u);
+    if (t == 0u) *word = 0u;
 #pragma unroll
     for (int v = 0; v < 4; ++v) red[wave * 256u + (uint32_t)v * 64u + lane] = acc[0][v] + acc[1][v];
     __syncthreads();
-    atomicMax(&mx[n], __float_as_uint(ma));
-    atomicMax(&mx[16u + n], __float_as_uint(mb));
-    __syncthreads();
-    if (t >= 256u) return;
-    float s = red[t];
+    float s = red[t & 255u];
 #pragma unroll
-    for (uint32_t w = 1; w < NWV; ++w) s += red[w * 256u + t];
+    for (uint32_t w = 1; w < NWV; ++w) s += red[w * 256u + (t & 255u)];
+    if ((lost & 0xFFFFu) != 0u || vx_gemm_bf_odd(s)) *word = 1u;
+    __syncthreads();
+    const bool look = *word != 0u;
+    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + 32;  // of each row of A and column of B, see vx_scan
+    if (look) {
+        if (t < 64u) mx[t] = 0u;
+        __syncthreads();
+        auto all = [](uint32_t) { return true; };
+        vx_scan<AM == MODE_K, 16>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NWV, lane, mx, ls, all);
+        vx_scan<BM == MODE_K, 16>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 16, ls + 16, all);
+        __syncthreads();
+    }
+    if (t >= 256u) return;
     const uint32_t rt = 4u * ((t & 63u) >> 4) + (t >> 6), ct = t & 15u;
     const uint32_t row = m0 + rt, col = n0 + ct;
     if (row >= p.M || col >= p.N) return;
-    const float rm = __uint_as_float(mx[rt]), cm = __uint_as_float(mx[16u + ct]);
-    const bool tiny = (rm * cm < 0x1p-80f || fminf(rm, cm) < 0x1p-109f) && rm > 0.f && cm > 0.f;
-    if (!(__builtin_fabsf(s) < __builtin_inff()) || tiny)
+    if (look && vx_gemm_bf_again(s, p.K, mx[rt], ls[rt] != 0u, mx[16u + ct], ls[16u + ct] != 0u))
         s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
     vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
 }

@@ -55,12 +55,14 @@ __device__ __forceinline__ void vx_split8(const float (&v)[8], u32x4 (&t)[NT]) {
                                : vx_pk_bf16(r[2 * i], r[2 * i + 1]);
 }
 
-// v[0..8) as three terms of packed bf16 rounded to nearest, largest first:
-// exact down to bf16's smallest subnormal, and with |second| <= 2^-8 |v| and
-// |third| <= 2^-16 |v| of either sign, so that in a product of two such sums
-// the three smallest of the nine terms are below 2^-24 of it and average out.
-// |v| above 3.39e38 rounds to an infinity.
-__device__ __forceinline__ void vx_split8_rne(const float (&v)[8], u32x4 (&t)[3]) {
+// v[0..8) as three terms of packed bf16 rounded to nearest, largest first, with
+// |second| <= 2^-8 |v| and |third| <= 2^-16 |v| of either sign, so that in a
+// product of two such sums the three smallest of the nine terms are below 2^-24
+// of it and average out. |v| above 3.39e38 rounds to an infinity. The three add
+// up to v exactly, except for bits of v below 2^-133, bf16's smallest number
+// (there are any only where |v| < 2^-110): `lost` then gets some of its low 16
+// bits set, and only then (the last remainder has 8 bits; NaNs apart).
+__device__ __forceinline__ void vx_split8_rne(const float (&v)[8], u32x4 (&t)[3], uint32_t& lost) {
     float r[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) r[i] = v[i];
@@ -70,9 +72,11 @@ __device__ __forceinline__ void vx_split8_rne(const float (&v)[8], u32x4 (&t)[3]
         for (int i = 0; i < 4; ++i) {
             const uint32_t h = vx_pk_bf16(r[2 * i], r[2 * i + 1]);
             t[k][i] = h;
+            if (k == 2) lost |= __float_as_uint(r[2 * i]) | __float_as_uint(r[2 * i + 1]);
             r[2 * i] -= __uint_as_float(h << 16);
             r[2 * i + 1] -= __uint_as_float(h & 0xFFFF0000u);
         }
+    asm("" : "+v"(lost));  // (formed here: left free, the compiler kept the remainders)
 }
 
 // A second look at those of the T rows (or columns) x0.. of an operand for which

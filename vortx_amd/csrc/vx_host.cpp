@@ -367,8 +367,8 @@ static int launch_gemm_bf(vx_ctx ctx, vx_stream stream, const vx_gemm_args& g, i
     // A / B with stride 1 along K: 16-byte loads along it (4-byte aligned: any row stride); else along M / N
     const int k = tab[g.as[3] == 1 ? 0 : 1][g.bs[2] == 1 ? 0 : 1][cfg];
     const uint32_t tm = kBfRows[cfg], tn = kBfCols[cfg];
-    // two buffers of a stage's terms (6 bytes an element) and a word; the K split: the waves' sums and 64 words
-    const size_t lds = cfg >= BF_KS ? 8u * tm * tn * 4u + (tm + tn) * 4u
+    // two buffers of a stage's terms (6 bytes an element), or the K split's partial sums of its waves, and a word
+    const size_t lds = cfg >= BF_KS ? 8u * tm * tn * 4u + 16u
                                     : (size_t)(tm + tn) * (cfg == BF_S2 ? 64u : 32u) * 12u + 16u;
     // a grid holds fewer than 2^32 threads: at most 2^21 tiles per launch
     const uint32_t sm = tm << 10, sn = tn << 11;
