@@ -46,3 +46,45 @@ def test_small_elements_beside_large_ones(gemm, M, N, K, ta, tb):
     ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
     err, bound = (c.double() - ref).abs(), (K + 32) * 2.0 ** -24 * mag + K * 2.0 ** -149
     assert bool((err <= bound).all()), f"{float((err / bound).max())} of the bound"
+
+
+def _us(f):
+    f()
+    best = float("inf")
+    for _ in range(5):
+        t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        t0.record()
+        f()
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1) * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)], ids=["ab", "aTbT"])
+@pytest.mark.parametrize("M,N,K", [(16, 1600, 4096), (300, 517, 4096), (1200, 1100, 1000), (970, 1000, 2000), (2100, 1900, 1000),
+                                   (4000, 4011, 1000)])
+def test_cost_of_non_finite_and_small(gemm, M, N, K, ta, tb):
+    """A NaN or an infinity in every row, or products far below one: what f32
+    products give, in a bounded time (measured up to 5.5 times an ordinary
+    call's; forming each output in one lane took 20 times and more)."""
+    note(f"gemm_bf cost {M}x{N}x{K} ta={ta} tb={tb}")
+    a, b = S.uniform((M, K), 1, DEV) + 2.0, S.uniform((K, N), 2, DEV)
+    a = a.t().contiguous().t() if ta else a
+    b = b.t().contiguous().t() if tb else b
+    c = torch.empty((M, N), device=DEV)
+    base = _us(lambda: gemm.dispatch_tiled(c, a, b))
+    rows = torch.arange(M, device=DEV)
+    for what in ("nan", "inf", "1e-13", "1e-20"):
+        aa, bb = (a * float(what), b * float(what)) if what[0] == "1" else (a.clone(), b)
+        if what[0] != "1":
+            aa[rows, rows % K] = float(what)
+        us = _us(lambda: gemm.dispatch_tiled(c, aa, bb))
+        note(f"  {what}: {us:.0f} us, {base:.0f} without")
+        ref = aa.double() @ bb.double()
+        if what[0] == "1":
+            bound = (K + 32) * 2.0 ** -24 * (aa.double().abs() @ bb.double().abs()) + K * 2.0 ** -149
+            assert bool(((c.double() - ref).abs() <= bound).all()), what
+        else:
+            assert torch.equal(c.isnan(), ref.isnan()) and torch.equal(c[ref.isinf()].double(), ref[ref.isinf()])
+        assert us < (2 if what == "1e-13" else 8) * base + 50, f"{what}: {us:.0f} us, {base:.0f} without"

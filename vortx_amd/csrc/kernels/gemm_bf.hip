@@ -100,27 +100,173 @@ struct vx_slab {
     }
 };
 
+// One operand's chunk of 32 elements of K of lane (n, g)'s x for the bf16 terms:
+// H pieces of 8 elements (H G = 4; 32 x 32 tiles: g 0..1; 16 x 16: g 0..3).
+template <int MODE, int H, int G>
+struct vx_chunk {
+    static constexpr uint32_t KC = 8u * G * H;
+    float r[H][8];
+    // where the lane's pieces of chunk 0 begin in its row or column p
+    static __device__ __forceinline__ const float* base(const float* p, int64_t sk, uint32_t g) { return p + (int64_t)(8u * g) * sk; }
+    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            if constexpr (MODE == MODE_K) {
+                const float* q = p + (k0 + 8u * G * h);
+                const f32x4_a4 a = *(const f32x4_a4*)q, b = *(const f32x4_a4*)(q + 4);
+                r[h][0] = a.x; r[h][1] = a.y; r[h][2] = a.z; r[h][3] = a.w;
+                r[h][4] = b.x; r[h][5] = b.y; r[h][6] = b.z; r[h][7] = b.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) r[h][j] = p[(int64_t)(k0 + 8u * G * h + (uint32_t)j) * sk];  // (a scalar offset)
+            }
+        }
+    }
+    __device__ __forceinline__ void load_tail(const float* p, int64_t sk, uint32_t k0, uint32_t g, uint32_t K) {
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t k = k0 + 8u * G * h + 8u * g + (uint32_t)j, kc = min(k, K - 1u);
+                const float e = p[((int64_t)kc - 8u * g) * (MODE == MODE_K ? 1 : sk)];  // (clamped: no branches between the loads)
+                r[h][j] = k < K ? e : 0.f;
+            }
+    }
+};
+
+// The same of 16 elements for f32 products in the order of K: step s of a product
+// takes element G s + g.
+template <int MODE, int G>
+struct vx_seq {
+    static constexpr uint32_t KC = 16u;
+    static constexpr int NS = 16 / G, NR = MODE == MODE_K ? 16 : NS;
+    float r[NR];
+    static __device__ __forceinline__ const float* base(const float* p, int64_t sk, uint32_t g) { return MODE == MODE_K ? p : p + (int64_t)g * sk; }
+    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0) {
+        if constexpr (MODE == MODE_K) {
+#pragma unroll
+            for (int j = 0; j < 16; j += 4) {
+                const f32x4_a4 a = *(const f32x4_a4*)(p + k0 + j);
+                r[j] = a.x; r[j + 1] = a.y; r[j + 2] = a.z; r[j + 3] = a.w;
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) r[s] = p[(int64_t)(k0 + (uint32_t)(G * s)) * sk];
+        }
+    }
+    __device__ __forceinline__ void load_tail(const float* p, int64_t sk, uint32_t k0, uint32_t g, uint32_t K) {
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            const uint32_t k = k0 + (MODE == MODE_K ? (uint32_t)j : (uint32_t)(G * j) + g), kc = min(k, K - 1u);
+            const float e = MODE == MODE_K ? p[kc] : p[((int64_t)kc - g) * sk];
+            r[j] = k < K ? e : 0.f;
+        }
+    }
+    __device__ __forceinline__ float at(int s, uint32_t g) const {
+        if constexpr (MODE != MODE_K) {
+            return r[s];
+        } else {
+            // (bit masks: a choice between array elements went through scratch memory)
+            float e = 0.f;
+#pragma unroll
+            for (uint32_t j = 0; j < (uint32_t)G; ++j) {
+                const uint32_t m = g == j ? ~0u : 0u;
+                e = __uint_as_float(__float_as_uint(e) | (__float_as_uint(r[G * s + j]) & m));
+            }
+            return e;
+        }
+    }
+};
+
+// K in chunks, chunks w, w + nw, ... of it to mult(a, b, odd chunk) straight
+// from memory (no LDS, no barrier, one chunk ahead): pa and pb point at element 0
+// of the lane's row of A and column of B.
+template <class CA, class CB, class Mult>
+__device__ __forceinline__ void vx_chunks(const vx_gemm_args& p, const float* pa, const float* pb, uint32_t g, uint32_t w, uint32_t nw,
+                                          const Mult& mult) {
+    constexpr uint32_t KC = CA::KC;
+    pa = CA::base(pa, p.as[3], g);
+    pb = CB::base(pb, p.bs[2], g);
+    const uint32_t nck = p.K / KC;  // whole chunks
+    if (w < nck) {
+        CA a[2];
+        CB b[2];
+        const uint32_t last = (nck - 1u - w) / nw * nw + w;  // this wave's last chunk
+        auto load = [&](int d, uint32_t c) {
+            a[d].load(pa, p.as[3], min(c, last) * KC);
+            b[d].load(pb, p.bs[2], min(c, last) * KC);
+        };
+        load(0, w);
+        load(1, w + nw);
+        uint32_t c = w;
+        for (; c + nw <= last; c += 2u * nw) {
+            // (each chunk's next loads go out as soon as it is split: left free,
+            // the compiler issued both chunks' at the end of the round)
+            __builtin_amdgcn_sched_barrier(0);
+            mult(a[0], b[0], 0);
+            load(0, c + 2u * nw);
+            __builtin_amdgcn_sched_barrier(0);
+            mult(a[1], b[1], 1);
+            load(1, c + 3u * nw);
+        }
+        if (c <= last) mult(a[0], b[0], 0);
+    }
+    if (p.K % KC != 0u && w == nck % nw) {
+        CA a;
+        CB b;
+        a.load_tail(pa, p.as[3], nck * KC, g, p.K);
+        b.load_tail(pb, p.bs[2], nck * KC, g, p.K);
+        mult(a, b, 1);
+    }
+}
+
+// 32 x 32 or 16 x 16 outputs of a wave as f32 multiply-adds from the first k to
+// the last, one rounding each: the f32 matrix cores add a step's products one
+// after another in the order of the lane groups g (so measured, bit for bit).
+// Where a sum overflows on the way, or infinities meet, this order decides; the
+// same one in every kernel.
+template <int AM, int BM>
+__device__ __forceinline__ void vx_f32_tile(const vx_gemm_args& p, const float* pa, const float* pb, uint32_t g, f32x16& acc) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    vx_chunks<vx_seq<AM, 2>, vx_seq<BM, 2>>(p, pa, pb, g, 0u, 1u, [&](const auto& a, const auto& b, int) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.at(s, g), b.at(s, g), acc, 0, 0, 0);
+    });
+}
+template <int AM, int BM>
+__device__ __forceinline__ void vx_f32_tile(const vx_gemm_args& p, const float* pa, const float* pb, uint32_t g, f32x4& acc) {
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    vx_chunks<vx_seq<AM, 4>, vx_seq<BM, 4>>(p, pa, pb, g, 0u, 1u, [&](const auto& a, const auto& b, int) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.at(s, g), b.at(s, g), acc, 0, 0, 0);
+    });
+}
+
 // Outputs of a tile that lost bits of an operand (vx_split8_rne), or that holds
 // an output for which odd() is true, are looked at again. The tile's rows of A
-// and columns of B are scanned (vx_scan), and an output is formed the plain way
+// and columns of B are scanned (vx_scan); where one holds a NaN, so does the
+// output. Any other is formed from f32 products (vx_f32_tile)
 //   where it is not finite: the terms of an infinity hold a NaN;
 //   where it is below 2^-120: its six sums would be rounded to 2^-149 each;
 //   where an element of its row or column misses bits, up to 2^-134 each, and
 //   they may count: K 2^-134 max|b| + K 2^-134 max|a| against 2^-24 of it.
 // (The matrix cores keep subnormal operands, products and sums.)
+// What this takes, us, without / a NaN in every row of A (the scan) / an infinity
+// in every row (all outputs formed again; bound by the f32 matrix cores and, in
+// the K split kernels, by one wave's loads): 4000 x 4011 x 1000 195 / 288 / 764,
+// 2100 x 1900 x 1000 60 / 87 / 241, 970 x 1000 x 2000 42 / 65 / 135, 300 x 517 x
+// 4096 32 / 52 / 173. One lane per output, in the same order of additions, took
+// 12000 to 36000 on the first with NaNs.
 __device__ __forceinline__ bool vx_gemm_bf_odd(float s) {
     const float v = __builtin_fabsf(s);
     return !(v < __builtin_inff()) || (v < 0x1p-120f && v > 0.f);
 }
-// ra, cb: the bits of the largest |a| of the row and |b| of the column
+// ra, cb: the bits of the largest |a| of the row and |b| of the column (a NaN's are larger)
 __device__ __forceinline__ bool vx_gemm_bf_again(float s, uint32_t K, uint32_t ra, bool rlost, uint32_t cb, bool clost) {
+    if (ra > 0x7F800000u || cb > 0x7F800000u) return false;
     const float big = fmaxf(rlost ? __uint_as_float(cb) : 0.f, clost ? __uint_as_float(ra) : 0.f);
     return vx_gemm_bf_odd(s) || ((rlost || clost) && !(__builtin_fabsf(s) >= (float)K * 0x1p-109f * big));
-}
-__device__ __forceinline__ float vx_gemm_bf_redo(const vx_gemm_args& p, const float* a, const float* b) {
-    float s = 0.f;
-    for (uint32_t k = 0; k < p.K; ++k) s = __builtin_fmaf(a[(int64_t)k * p.as[3]], b[(int64_t)k * p.bs[2]], s);
-    return s;
 }
 
 extern __shared__ __align__(16) uint8_t vx_bf_lds[];
@@ -350,31 +496,31 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
         __syncthreads();
     }
     if (wh) return;
-    uint64_t again = 0;  // outputs to form the plain way
-    static_assert(MI * NJ * 16 <= 64, "one bit per output of a lane");
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const uint32_t ct = ct0 + 32u * j;
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i) {
+            float* c1 = c0 + (int64_t)(32 * i) * p.cs[2] + (int64_t)(32 * j) * p.cs[3];
+            uint32_t again = 0u;  // outputs to form from f32 products
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const uint32_t rt = rt0 + 32u * i + 8u * (v >> 2) + (v & 3);
                 if (m0 + rt < p.M && n0 + ct < p.N) {
                     if (!look || !vx_gemm_bf_again(acc[0][i][j][v], p.K, mx[rt], ls[rt] != 0u, mx[TM + ct], ls[TM + ct] != 0u))
-                        vx_epilogue(c0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * p.cs[2] + (int64_t)(32 * j) * p.cs[3],
-                                    acc[0][i][j][v], p.alpha, p.beta);
+                        vx_epilogue(c1 + (int64_t)(8 * (v >> 2) + (v & 3)) * p.cs[2], acc[0][i][j][v], p.alpha, p.beta);
                     else
-                        again |= 1ull << ((j * MI + i) * 16 + v);
+                        again |= 1u << v;
                 }
             }
-    }
-    while (again) {
-        const uint32_t o = (uint32_t)__builtin_ctzll(again), v = o & 15u, i = (o >> 4) % MI, j = (o >> 4) / MI;
-        again &= again - 1u;
-        const uint32_t row = m0 + rt0 + 32u * i + 8u * (v >> 2) + (v & 3u), col = n0 + ct0 + 32u * j;
-        const float s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
-        vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+            if (!__any(again != 0u)) continue;
+            f32x16 f;
+            vx_f32_tile<AM, BM>(p, A + (int64_t)min(m0 + wm * (32u * MI) + 32u * i + n, p.M - 1u) * p.as[2],
+                                B + (int64_t)min(n0 + ct, p.N - 1u) * p.bs[3], g, f);
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (again >> v & 1u) vx_epilogue(c1 + (int64_t)(8 * (v >> 2) + (v & 3)) * p.cs[2], f[v], p.alpha, p.beta);
+        }
     }
 }
 
@@ -383,35 +529,6 @@ __device__ __forceinline__ void vx_gemm_bf(const vx_gemm_args& p) {
 // small output from a long K). Wave w takes the 32-element chunks w, w + 8, ...
 // of K straight from memory to registers (no LDS, no barrier in the loop, one
 // chunk ahead), and the waves' sums meet in LDS in wave order.
-template <int MODE>
-struct vx_chunk {  // one operand's 32 k of lane (n, g)'s x: k16 step h, elements 8g..8g+7
-    float r[2][8];
-    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0, uint32_t g) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t k = k0 + 16u * h + 8u * g;
-            if constexpr (MODE == MODE_K) {
-                const f32x4_a4 a = *(const f32x4_a4*)(p + k), b = *(const f32x4_a4*)(p + k + 4);
-                r[h][0] = a.x; r[h][1] = a.y; r[h][2] = a.z; r[h][3] = a.w;
-                r[h][4] = b.x; r[h][5] = b.y; r[h][6] = b.z; r[h][7] = b.w;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) r[h][j] = p[(int64_t)(k + (uint32_t)j) * sk];
-            }
-        }
-    }
-    __device__ __forceinline__ void load_tail(const float* p, int64_t sk, uint32_t k0, uint32_t g, uint32_t K) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t k = k0 + 16u * h + 8u * g + (uint32_t)j, kc = min(k, K - 1u);
-                const float e = p[MODE == MODE_K ? (int64_t)kc : (int64_t)kc * sk];  // (clamped: no branches between the loads)
-                r[h][j] = k < K ? e : 0.f;
-            }
-    }
-};
-
 template <int AM, int BM>
 __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
     constexpr uint32_t NWV = 8;
@@ -432,7 +549,7 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.f;
     uint32_t lost = 0u;  // see vx_split8_rne
-    auto mult = [&](const vx_chunk<AM>& a, const vx_chunk<BM>& b) {
+    auto mult = [&](const auto& a, const auto& b, int) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             u32x4 ta[3], tb[3];
@@ -445,37 +562,7 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
                                                                  __builtin_bit_cast(bf16x8, tb[TB[e]]), acc[h], 0, 0, 0);
         }
     };
-    const uint32_t nck = p.K / 32u;  // whole chunks
-    if (wave < nck) {
-        vx_chunk<AM> a[2];
-        vx_chunk<BM> b[2];
-        const uint32_t last = (nck - 1u - wave) / NWV * NWV + wave;  // this wave's last chunk
-        auto load = [&](int d, uint32_t c) {
-            a[d].load(pa, p.as[3], min(c, last) * 32u, g);
-            b[d].load(pb, p.bs[2], min(c, last) * 32u, g);
-        };
-        load(0, wave);
-        load(1, wave + NWV);
-        uint32_t c = wave;
-        for (; c + NWV <= last; c += 2u * NWV) {
-            // (each chunk's next loads go out as soon as it is split: left free,
-            // the compiler issued both chunks' at the end of the round)
-            __builtin_amdgcn_sched_barrier(0);
-            mult(a[0], b[0]);
-            load(0, c + 2u * NWV);
-            __builtin_amdgcn_sched_barrier(0);
-            mult(a[1], b[1]);
-            load(1, c + 3u * NWV);
-        }
-        if (c <= last) mult(a[0], b[0]);
-    }
-    if (p.K % 32u != 0u && wave == nck % NWV) {
-        vx_chunk<AM> a;
-        vx_chunk<BM> b;
-        a.load_tail(pa, p.as[3], nck * 32u, g, p.K);
-        b.load_tail(pb, p.bs[2], nck * 32u, g, p.K);
-        mult(a, b);
-    }
+    vx_chunks<vx_chunk<AM, 2, 2>, vx_chunk<BM, 2, 2>>(p, pa, pb, g, wave, NWV, mult);
     // red[wave][v][lane], and whether the tile needs a closer look
     float* red = (float*)vx_bf_lds;
     uint32_t* word = (uint32_t*)(red + NWV * 1024u);
@@ -502,14 +589,33 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
         vx_scan<BM == MODE_K, 32>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 32, ls + 32, all);
         __syncthreads();
     }
+    bool again[2] = {false, false};  // outputs to form from f32 products
+    const uint32_t rt0 = 8u * (t >> 8) + 4u * (lane >> 5) + (wave & 3u), ct = lane & 31u;  // output u: row rt0 + 16 u, column ct
+    if (look) {
+#pragma unroll
+        for (uint32_t u = 0; u < 2u; ++u)
+            again[u] = vx_gemm_bf_again(s[u], p.K, mx[rt0 + 16u * u], ls[rt0 + 16u * u] != 0u, mx[32u + ct], ls[32u + ct] != 0u);
+        if (again[0] || again[1]) *word = 2u;
+        __syncthreads();
+        if (*word == 2u) {
+            if (wave < 4u) {  // 16 x 16 outputs each
+                const uint32_t r0 = 16u * (wave >> 1), c0 = 16u * (wave & 1u), n16 = lane & 15u, g4 = lane >> 4;
+                f32x4 f;
+                vx_f32_tile<AM, BM>(p, A + (int64_t)min(m0 + r0 + n16, p.M - 1u) * p.as[2],
+                                    B + (int64_t)min(n0 + c0 + n16, p.N - 1u) * p.bs[3], g4, f);
+#pragma unroll
+                for (uint32_t v = 0; v < 4u; ++v) red[(r0 + 4u * g4 + v) * 32u + c0 + n16] = f[v];
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < 2u; ++u)
+                if (again[u]) s[u] = red[(rt0 + 16u * u) * 32u + ct];
+        }
+    }
 #pragma unroll
     for (uint32_t u = 0; u < 2u; ++u) {
-        const uint32_t o = t + 512u * u, l = o & 63u, v = o >> 6, rt = 8u * (v >> 2) + 4u * (l >> 5) + (v & 3u), ct = l & 31u;
-        const uint32_t row = m0 + rt, col = n0 + ct;
-        if (row >= p.M || col >= p.N) continue;
-        if (look && vx_gemm_bf_again(s[u], p.K, mx[rt], ls[rt] != 0u, mx[32u + ct], ls[32u + ct] != 0u))
-            s[u] = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
-        vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s[u], p.alpha, p.beta);
+        const uint32_t row = m0 + rt0 + 16u * u, col = n0 + ct;
+        if (row < p.M && col < p.N) vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s[u], p.alpha, p.beta);
     }
 }
 
@@ -525,30 +631,6 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
 // waves (44.4, 47.2 us on the first), three or four chunks ahead (no gain), 32 x
 // 16 tiles (46.3; 31 x 4096 x 4096 25.6 against 33.7 and 34.5, the only size
 // where they won).
-template <int MODE>
-struct vx_strip {  // one operand's 32 k of lane (n, g)'s x: elements 8g..8g+7
-    float r[8];
-    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0, uint32_t g) {
-        const uint32_t k = k0 + 8u * g;
-        if constexpr (MODE == MODE_K) {
-            const f32x4_a4 a = *(const f32x4_a4*)(p + k), b = *(const f32x4_a4*)(p + k + 4);
-            r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
-            r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) r[j] = p[(int64_t)(k + (uint32_t)j) * sk];
-        }
-    }
-    __device__ __forceinline__ void load_tail(const float* p, int64_t sk, uint32_t k0, uint32_t g, uint32_t K) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t k = k0 + 8u * g + (uint32_t)j, kc = min(k, K - 1u);
-            const float e = p[MODE == MODE_K ? (int64_t)kc : (int64_t)kc * sk];  // (clamped: no branches between the loads)
-            r[j] = k < K ? e : 0.f;
-        }
-    }
-};
-
 template <int AM, int BM>
 __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
     constexpr uint32_t NWV = 8;
@@ -566,45 +648,17 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
 
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // even and odd chunks
     uint32_t lost = 0u;  // see vx_split8_rne
-    auto mult = [&](const vx_strip<AM>& a, const vx_strip<BM>& b, int par) {
+    auto mult = [&](const auto& a, const auto& b, int par) {
         u32x4 ta[3], tb[3];
-        vx_split8_rne(a.r, ta, lost);
-        vx_split8_rne(b.r, tb, lost);
+        vx_split8_rne(a.r[0], ta, lost);
+        vx_split8_rne(b.r[0], tb, lost);
         constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};  // smallest products first
 #pragma unroll
         for (int e = 0; e < 6; ++e)
             acc[par] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ta[TA[e]]),
                                                                __builtin_bit_cast(bf16x8, tb[TB[e]]), acc[par], 0, 0, 0);
     };
-    const uint32_t nck = p.K / 32u;  // whole chunks
-    if (wave < nck) {
-        vx_strip<AM> a[2];
-        vx_strip<BM> b[2];
-        const uint32_t last = (nck - 1u - wave) / NWV * NWV + wave;  // this wave's last chunk
-        auto load = [&](int d, uint32_t c) {
-            a[d].load(pa, p.as[3], min(c, last) * 32u, g);
-            b[d].load(pb, p.bs[2], min(c, last) * 32u, g);
-        };
-        load(0, wave);
-        load(1, wave + NWV);
-        uint32_t c = wave;
-        for (; c + NWV <= last; c += 2u * NWV) {
-            __builtin_amdgcn_sched_barrier(0);  // (as in vx_gemm_bf_ks)
-            mult(a[0], b[0], 0);
-            load(0, c + 2u * NWV);
-            __builtin_amdgcn_sched_barrier(0);
-            mult(a[1], b[1], 1);
-            load(1, c + 3u * NWV);
-        }
-        if (c <= last) mult(a[0], b[0], 0);
-    }
-    if (p.K % 32u != 0u && wave == nck % NWV) {
-        vx_strip<AM> a;
-        vx_strip<BM> b;
-        a.load_tail(pa, p.as[3], nck * 32u, g, p.K);
-        b.load_tail(pb, p.bs[2], nck * 32u, g, p.K);
-        mult(a, b, 1);
-    }
+    vx_chunks<vx_chunk<AM, 1, 4>, vx_chunk<BM, 1, 4>>(p, pa, pb, g, wave, NWV, mult);
     // red[wave][v][lane], and whether the tile needs a closer look
     float* red = (float*)vx_bf_lds;
     uint32_t* word = (uint32_t*)(red + NWV * 256u);
@@ -627,13 +681,24 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
         vx_scan<BM == MODE_K, 16>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 16, ls + 16, all);
         __syncthreads();
     }
-    if (t >= 256u) return;
-    const uint32_t rt = 4u * ((t & 63u) >> 4) + (t >> 6), ct = t & 15u;
+    const uint32_t rt = 4u * (lane >> 4) + (wave & 3u), ct = lane & 15u;  // of the first four waves' outputs
+    if (look) {
+        const bool again = vx_gemm_bf_again(s, p.K, mx[rt], ls[rt] != 0u, mx[16u + ct], ls[16u + ct] != 0u);
+        if (again) *word = 2u;
+        __syncthreads();
+        if (*word == 2u) {
+            if (wave == 0u) {
+                f32x4 f;
+                vx_f32_tile<AM, BM>(p, pa, pb, g, f);
+#pragma unroll
+                for (uint32_t v = 0; v < 4u; ++v) red[v * 64u + lane] = f[v];
+            }
+            __syncthreads();
+            if (again) s = red[t & 255u];
+        }
+    }
     const uint32_t row = m0 + rt, col = n0 + ct;
-    if (row >= p.M || col >= p.N) return;
-    if (look && vx_gemm_bf_again(s, p.K, mx[rt], ls[rt] != 0u, mx[16u + ct], ls[16u + ct] != 0u))
-        s = vx_gemm_bf_redo(p, A + (int64_t)row * p.as[2], B + (int64_t)col * p.bs[3]);
-    vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+    if (t < 256u && row < p.M && col < p.N) vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
 }
 
 // 256 x 128 tiles (8 waves of 64 x 64), 128 x 128 (2 x 4 waves of 64 x 64) and

@@ -112,7 +112,15 @@ __device__ __forceinline__ void vx_scan(const float* base, int64_t sx, int64_t s
 #pragma unroll
             for (int j = 0; j < 16; ++j) take(v[j]);
         }
-        for (k += k0; k < K; k += step) take(p[(int64_t)k * ks]);
+        if (k < K) {  // (past K the last element again: no branches between the loads)
+            const uint32_t rem = (uint32_t)(K - k) - 1u;
+            q = p + (int64_t)k * ks;
+            float v[16];
+#pragma unroll
+            for (uint32_t j = 0; j < 16u; ++j) v[j] = q[(int64_t)min(k0 + j * step, rem) * ks];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) take(v[j]);
+        }
         if constexpr (KC) {
 #pragma unroll
             for (int o = 32; o; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
