@@ -250,8 +250,11 @@ int vx_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y,
  * 1.6e-5 max|x_block|; products and block sums with the exactly decoded
  * weights are exact in int32 and the scaling is f32. Batch 1 reduces with
  * v_dot4_i32_i8, batches (B >= 2) on the int8 matrix cores. VX_GEMV_X_F32
- * keeps x in f32 instead (on the exactly decoded weights; slower);
- * VX_GEMV_X_INT8 names the default split and may not be combined with it. */
+ * keeps x in f32 instead (on the exactly decoded weights; slower).
+ * VX_GEMV_X_INT8 asks for the split at every shape (the default may take two
+ * bf16 terms for many columns, see vx_gemv_q): the results are those of
+ * vx_quantize_x and vx_gemv_q_xq, bit for bit. It may not be combined with
+ * VX_GEMV_X_F32. */
 typedef enum vx_gemv_flags { VX_GEMV_X_INT8 = 1, VX_GEMV_X_F32 = 2 } vx_gemv_flags;
 /* With VX_GEMV_X_INT8, a batched shape whose split needs device memory
  * (see vx_gemv_q) returns VX_ERR_UNSUPPORTED here instead of falling back
@@ -265,8 +268,9 @@ int vx_gemv_q_ex(vx_ctx ctx, vx_stream stream, const vx_mview* y,
  * (src/linalg/gemm.rs:47-56): per-caller mutable state kept outside the
  * (immutable) context. Where a batched call needs its activation split in
  * memory (see vx_gemv_q), x is split into `workspace` by the vx_quantize_x
- * kernel and the GEMV reads it (two launches on `stream`); elsewhere, many
- * columns (vx_gemv_q) among it, the workspace is not touched. workspace: device memory, 16-byte aligned, at
+ * kernel and the GEMV reads it (two launches on `stream`); elsewhere (many
+ * columns on two bf16 terms, see vx_gemv_q, among it) the workspace is not
+ * touched. workspace: device memory, 16-byte aligned, at
  * least vx_gemv_q_ws_size(...) bytes (a smaller non-NULL workspace is
  * VX_ERR_INVALID; NULL behaves as vx_gemv_q_ex). The library never
  * allocates, frees or retains it; its contents need not start at zero.
@@ -336,13 +340,14 @@ int vx_gemv_q_xq(vx_ctx ctx, vx_stream stream, const vx_mview* y,
 /* vx_gemv_q_ws without a caller workspace, allocating nothing. No
  * counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc) yet want the int8 split at every batched shape. Same
+ * forbid hipMalloc) yet want the routes that need a workspace. Same
  * arguments and flags as vx_gemv_q_ex, and the kernels and results of
  * vx_gemv_q_ws: where that one splits x into the caller's workspace
  * (B >= 2), this one uses a fixed
  * device array of VX_NOALLOC_SCRATCH_BYTES (4 MiB) that the library's GEMV
  * code object holds per context from vx_init to vx_destroy, so the split of
- * x, vx_xq_size(K, B) bytes (72 per 32 elements of x), must fit it (else
+ * x, vx_xq_size(K, B) bytes (72 per 32 elements of x), must fit it, whether or
+ * not many columns then take the route without it (else
  * VX_ERR_UNSUPPORTED, nothing launched): B = 16 up to K = 116480, B = 64 up
  * to K = 28928. Every call on
  * one context uses the same array: calls that overlap in time on one

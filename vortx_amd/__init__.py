@@ -377,12 +377,15 @@ class QuantGemv(_Context):
                  workspace=None) -> None:
         """y = W x. By default x is split per 32-block into two int8 levels
         (error <= 1.6e-5 of the block's max|x|) and every product is exact in
-        int32 (include/vortx_hip.h, vx_gemv_q_ex). ``x_f32=True`` keeps x in
-        f32 (f32 FMA on the exactly decoded weights); ``x_int8=True`` names
-        the default explicitly. ``workspace``: a uint8 GPU tensor of at least
-        ``workspace_size(w, B)`` bytes (vx_gemv_q_ws), where batched shapes
-        split x when the GEMV kernel cannot split it itself; without one
-        those shapes keep x in f32 (or, with ``x_int8``, raise)."""
+        int32; more than 16 columns with a workspace may take x as two bf16
+        terms instead (error <= 2^-16 |x|; include/vortx_hip.h, vx_gemv_q).
+        ``x_f32=True`` keeps x in f32 (up to four columns f32 FMA on the
+        exactly decoded weights, more of them three bf16 terms whose sum is
+        x); ``x_int8=True`` asks for the int8 split at every shape.
+        ``workspace``: a uint8 GPU tensor of at least ``workspace_size(w, B)``
+        bytes (vx_gemv_q_ws), where batched shapes split x when the GEMV
+        kernel cannot split it itself; without one those shapes keep x in f32
+        (or, with ``x_int8``, raise)."""
         flags = (_ffi.VX_GEMV_X_F32 if x_f32 else 0) | (_ffi.VX_GEMV_X_INT8 if x_int8 else 0)
         st = _pycall.gemv(_GEMV_EX, _GEMV_WS, self._ctx, stream, y, w, x, flags, workspace)
         if st is not None:

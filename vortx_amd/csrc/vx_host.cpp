@@ -1019,9 +1019,10 @@ static int run_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y, const vx_
                 std::to_string(nb) + " bytes of device memory: pass a workspace (vx_gemv_q_ws)";
             return fail(VX_ERR_UNSUPPORTED, m.c_str());
         }
-        if (q.base && B > 16u && gemm_q_ok(w)) {
+        if (q.base && B > 16u && !(flags & VX_GEMV_X_INT8) && gemm_q_ok(w)) {
             // two bf16 terms of x are closer to it than the int8 split, and
-            // W streams once per tile of columns instead of once per 16
+            // W streams once per tile of columns instead of once per 16 (a
+            // caller that names the int8 split gets it)
             double us = 0.0;
             const int cfg = gemm_q_choose(ctx, w->qtype, M, K, B, 2, &us);
             if (us < gemv_xq_us(w->qtype, M, K, B)) return launch_gemm_q(ctx, stream, cy, w, cx, B, 2, cfg);
