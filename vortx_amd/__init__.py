@@ -22,6 +22,7 @@ fallback.
 from __future__ import annotations
 
 import ctypes as C
+import warnings
 from dataclasses import dataclass
 
 from . import _ffi
@@ -37,8 +38,16 @@ lib()
 
 # Calls with plain torch tensors build their views in C (csrc/vx_pycall.cpp);
 # those functions return None for anything else, which then takes the ctypes
-# path below.
-from . import _pycall  # noqa: E402
+# path below. A Python that the extension was not built for takes that path for
+# every call.
+try:
+    from . import _pycall  # noqa: E402
+except ImportError:
+    warnings.warn("vortx_amd._pycall is not built for this Python: calls take the slower ctypes path", RuntimeWarning,
+                  stacklevel=2)
+
+    class _pycall:
+        gemm = gemv = quantize = dequantize = contiguous = setup = staticmethod(lambda *args: None)
 
 _ADDR = {name: C.cast(getattr(lib(), name), C.c_void_p).value
          for name in ("vx_gemm_f32", "vx_gemm_f32_ex", "vx_gemv_q_ex", "vx_gemv_q_ws", "vx_dequantize", "vx_quantize",

@@ -7,7 +7,7 @@ Steps (no cmake):
      library carries them and vx_init can hipModuleLoadData them;
   3. g++ for the host sources (HIP runtime API only), linked against
      libamdhip64;
-  4. g++ for the CPython extension with the binding's fast calls (_pycall.so).
+  4. g++ for the CPython extension with the binding's fast calls (_pycall.*.so).
 
 Every call recompiles everything (a build check, not an incremental build).
 """
@@ -25,7 +25,8 @@ INCLUDE = os.path.join(os.path.dirname(PKG), "include")  # the public C ABI head
 CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libvortx_hip.so")
-PYCALL = os.path.join(PKG, "_pycall.so")
+# named for the Python that it is built for: another one must not load it
+PYCALL = os.path.join(PKG, "_pycall" + sysconfig.get_config_var("EXT_SUFFIX"))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 
@@ -89,6 +90,9 @@ def build(verbose: bool = False) -> str:
           "-Wno-missing-field-initializers", f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}",
           os.path.join(CSRC, "vx_pycall.cpp"), "-o", tmp])
     os.replace(tmp, PYCALL)
+    untagged = os.path.join(PKG, "_pycall.so")  # from an older build
+    if os.path.exists(untagged):
+        os.remove(untagged)
     if verbose:
         print(f"built {LIB}")
     return LIB

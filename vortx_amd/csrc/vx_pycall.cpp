@@ -1,5 +1,5 @@
 // vx_pycall.cpp — the Python binding's calls with torch tensors, as a CPython
-// extension (vortx_amd/_pycall.so).
+// extension (vortx_amd/_pycall.<Python's tag>.so).
 //
 // Building the views of a call with ctypes structures took about 9 us of
 // host time a call; reading the tensors' attributes through the C API instead
