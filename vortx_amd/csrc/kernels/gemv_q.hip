@@ -1366,6 +1366,7 @@ __device__ __align__(256) uint8_t vx_scratch[VX_SCRATCH_BYTES];
 #define VX_XQ_FX_FLOAT2 192u
 template <int QT, int NCG, int XI, int RD, bool MP, bool ST, bool FX, bool FH, bool XM = false>
 __device__ __forceinline__ void vx_gemv_xq(const vx_gemv_xq_args& a) {
+    static_assert(!(MP && FX), "x is split in the kernel for one pass only");
     constexpr int NW = vx_unit<QT>::NW;
     constexpr uint32_t CP = 8u * NCG;             // columns per launch (padded)
     constexpr uint32_t PI = 16u * XI;             // items per pass
@@ -1689,13 +1690,9 @@ __device__ __forceinline__ void vx_gemv_xq(const vx_gemv_xq_args& a) {
         const uint32_t p = MP ? w / nts : 0u, ts = MP ? w - p * nts : w;
         if constexpr (MP) {
             if (ts == 0u && p > 0u) {
-                if constexpr (FX) {
-                    pass_split(p);
-                } else {
-                    pass_loads(p);
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    pass_publish(p);
-                }
+                pass_loads(p);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                pass_publish(p);
             }
         }
         (void)ts;
