@@ -33,10 +33,15 @@ def _check(c, a, b, K, what, alpha=1.0, beta=0.0, c0=None):
 
 
 # (M, N, K, batch): around 32 (the K split), 64, 128 and 256 (the tiles), K
-# around 32, 64 and 256 (stages, chunks of a wave); the last ones have outputs
-# enough for the tiles: 64 x 64 with long and short stages, 128 x 128, 256 x 128
+# around 32, 64 and 256 (stages, chunks of a wave). Kernels on 256 CUs
+# (tests/test_kernel_choice.py): k16 up to 100 x 70, then 64 x 64 with short
+# stages, twice, 128 x 128, 256 x 128; 64 x 64 with long stages (an odd and an
+# even number of them, with and without a tail), ks (with a tail, whole, a tail
+# alone on a wave), 256 x 128 twice
 SHAPES = [(32, 32, 64, 1), (31, 33, 31, 1), (33, 95, 257, 2), (1, 64, 4097, 1), (64, 1, 65, 3), (100, 70, 8, 1),
-          (1000, 1030, 161, 1), (1111, 1200, 192, 1), (2100, 1900, 170, 1), (1300, 1100, 130, 12)]
+          (1000, 1030, 161, 1), (1111, 1200, 192, 1), (2100, 1900, 170, 1), (1300, 1100, 130, 12),
+          (970, 1000, 673, 1), (1000, 1001, 1023, 1), (1000, 1003, 768, 1), (300, 517, 609, 1), (513, 301, 768, 1), (300, 517, 257, 1),
+          (4000, 4011, 500, 1), (2048, 4096, 333, 1)]
 
 
 @pytest.mark.parametrize("M,N,K,batch", SHAPES, ids=[f"{m}x{n}x{k}-{b}" for m, n, k, b in SHAPES])
@@ -59,7 +64,8 @@ def test_gemm_bf(gemm, M, N, K, batch, ta, tb):
         _check(c1, a, b, K, "alpha, beta", -0.5, 2.0, c0)
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 320, 500), (1500, 1333, 200), (2048, 2048, 160)])
+# small: 64 x 64 with long stages, short ones, short ones
+@pytest.mark.parametrize("M,N,K", [(970, 1000, 673), (1500, 1333, 200), (2048, 2048, 160)])
 def test_tile_shapes_give_the_same_bits(gemm, M, N, K):
     note(f"gemm_bf tiles {M}x{N}x{K}")
     a, b = S.uniform((M, K), 1, DEV), S.uniform((N, K), 2, DEV).t()
@@ -73,13 +79,18 @@ def test_tile_shapes_give_the_same_bits(gemm, M, N, K):
         assert torch.equal(_bits(c), _bits(out[0]))
 
 
-@pytest.mark.parametrize("M,N,K", [(70, 80, 300), (1200, 1100, 300)], ids=["k-split", "tiles"])
+# k16, ks, 64 x 64 with short and long stages, 128 x 128, 256 x 128
+KERNELS = pytest.mark.parametrize("M,N,K", [(70, 80, 300), (300, 517, 600), (1200, 1100, 300), (970, 1000, 673), (2100, 1900, 170),
+                                            (4000, 4011, 500)], ids=["k16", "ks", "s", "s2", "n", "w"])
+
+
+@KERNELS
 def test_non_finite_operands(gemm, M, N, K):
     """Infinities keep their sign, NaNs stay where they belong, and the largest
     finite floats are not taken for infinities."""
     note(f"gemm_bf non-finite {M}x{N}x{K}")
     a, b = S.uniform((M, K), 3, DEV) + 2.0, S.uniform((K, N), 4, DEV)
-    a[3, 17], a[5, K - 1], b[200, 9] = float("inf"), float("nan"), -float("inf")
+    a[3, 17], a[5, K - 1], b[min(200, K - 2), 9] = float("inf"), float("nan"), -float("inf")
     a[7, :], b[0, 11] = 0.0, torch.finfo(torch.float32).max
     a[8, :] = 0.0
     a[8, 0] = 0.5
@@ -99,7 +110,7 @@ def test_non_finite_operands(gemm, M, N, K):
     assert torch.isfinite(c[12:, 12:]).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(70, 80, 300), (1200, 1100, 300)], ids=["k-split", "tiles"])
+@KERNELS
 @pytest.mark.parametrize("ea,eb", [(-120, 60), (-60, -50), (-100, -30), (70, 40)])
 def test_far_from_one(gemm, M, N, K, ea, eb):
     """Operands whose smaller terms would fall below bf16's or f32's smallest

@@ -38,10 +38,13 @@ def _check(y, ref, mag, K, exact_x, what):
 
 
 # (rows, K, columns): one row and column tile of each K-split kernel and their
-# neighbours, partial items (K % 256 = 64, 128, 192), one unit; the last two
-# have enough outputs for the 256 x 128 tiles (whole items and a partial one)
+# neighbours, partial items (K % 256 = 64, 128, 192), one unit; then outputs
+# enough for the 256 x 128 tiles, of Q4_0 and Q4_K (whole items and a partial one)
+# and of Q8_0 too (whole items, and every partial one); 64 x 16 and 64 x 32 tiles
+# (tests/test_kernel_choice.py)
 SHAPES = [(1, 64, 17), (31, 256, 17), (33, 320, 33), (64, 512, 16), (65, 704, 65), (255, 192, 31), (1000, 128, 40),
-          (2049, 768, 1601), (2300, 320, 1500)]
+          (2049, 768, 1601), (2300, 320, 1500), (2300, 512, 1901), (2301, 576, 1900), (2299, 384, 1901), (2300, 448, 1902),
+          (8000, 256, 17), (8001, 448, 17), (8100, 512, 60), (8095, 320, 63)]
 
 
 @pytest.mark.parametrize("qtype", QTYPES, ids=lambda q: QN[q])
@@ -70,7 +73,7 @@ def test_many_columns(qgemv, qtype, M, K, B, exact_x):
 
 
 @pytest.mark.parametrize("qtype", QTYPES, ids=lambda q: QN[q])
-@pytest.mark.parametrize("M,B", [(70, 9), (2100, 1600)], ids=["k-split", "tiles"])
+@pytest.mark.parametrize("M,B", [(70, 9), (2100, 1600), (2300, 1901)], ids=["k-split", "tiles", "tiles-q8_0"])
 def test_non_finite_x_exact(qgemv, qtype, M, B):
     """With x kept in f32 an infinity or a NaN gives what the f32 products
     give (infinities keep their sign), in its own column only; the largest

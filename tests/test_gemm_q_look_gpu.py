@@ -52,7 +52,7 @@ def _us(f):
 
 
 @QTYPES
-@pytest.mark.parametrize("M,B", [(2000, 40), (2300, 1500)])
+@pytest.mark.parametrize("M,B", [(2000, 40), (2300, 1901)])
 def test_cost_of_non_finite_x(qgemv, qtype, M, B):
     """A NaN or an infinity in every column, or only zeros: the outputs of the f32 products,
     and a bounded time (measured 1.4 times an ordinary x's with NaNs or zeros, 3 to 6
@@ -77,7 +77,7 @@ def test_cost_of_non_finite_x(qgemv, qtype, M, B):
 
 
 @QTYPES
-@pytest.mark.parametrize("M,B", [(300, 9), (2300, 1500)])
+@pytest.mark.parametrize("M,B", [(300, 9), (2300, 1901)])
 @pytest.mark.parametrize("e", [-116, -122, -131])
 def test_small_x_keeps_its_bits(qgemv, qtype, M, B, e):
     """x kept in f32 far below one (its third terms would fall below bf16's
@@ -100,7 +100,7 @@ def test_small_x_keeps_its_bits(qgemv, qtype, M, B, e):
 
 
 @QTYPES
-@pytest.mark.parametrize("M,B", [(300, 40), (2300, 1500)])
+@pytest.mark.parametrize("M,B", [(300, 40), (2300, 1901)])
 def test_large_x_with_a_workspace(qgemv, qtype, M, B):
     """x around 1e37 with a workspace: a block's whole-number sum (up to 32 x 127
     times x) is beyond the largest float, the result is not."""

@@ -702,8 +702,8 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
 }
 
 // 256 x 128 tiles (8 waves of 64 x 64), 128 x 128 (2 x 4 waves of 64 x 64) and
-// 64 x 64 (2 x 4 waves of 32 x 32): _s up to three workgroups per CU, _s2 one,
-// with half the barriers.
+// 64 x 64 (2 x 4 waves of 32 x 32): _s two workgroups per CU, _s2 one, with half
+// the barriers.
 #define VX_GEMM_BF1(AM, BM, NAME, WPE, ...)                                                              \
     extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, WPE)))            \
     void vx_gemm_bf_##NAME(vx_gemm_args p) {                                                             \

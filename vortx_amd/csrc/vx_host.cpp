@@ -329,20 +329,27 @@ static int operand_mode(const Canon& c, int kdim, int xdim, uint32_t nb, uint32_
 // The bf16 matrix-core GEMM (gemm_bf.hip): tile shapes and the K split.
 enum BfCfg { BF_W = 0, BF_N = 1, BF_S2 = 2, BF_S = 3, BF_KS = 4, BF_K16 = 5 };
 static const uint32_t kBfRows[6] = {256, 128, 64, 64, 32, 16}, kBfCols[6] = {128, 128, 64, 64, 32, 16};
-// Choice by estimated time in us, rounds of resident workgroups times what a
-// round costs: a fixed part (first loads, last stores) and one per 32 elements
-// of K. Measured (graph-replayed): 256 x 128 tiles 8 + 2.55 (4096^3 2 rounds
-// 650 us, 1024 x 1024 x 128, batch 32 4 rounds 74 us), 128 x 128 5.4 + 1.34
-// (2048^3 one round 91 us, 4096^3 four 690 us), 64 x 64 with long stages 2.8 +
-// 0.6 (1024^3 one round 23.5 us), with short ones, three per CU, per tile of a
-// CU 1 + 0.45 (1000 x 1111 x 777 31 us, against 42 with long stages); the K
-// split 2 + 1.9 per 256 elements (8 x 11008 x 4096 two rounds 50 us, 1024^3
-// four 39 us, 256^3 one 6.6 us); in 16 x 16 tiles, several on a CU, 2.2 and per
-// tile of a CU 0.4 + 1 per 256 (8 x 11008 x 4096 44 us, 512^3 12.2, 256^3 4.1,
-// 16 x 4096 x 4096 17.5 to 19.5). tiles(tm, tn): tiles of that size.
+// Choice by estimated time in us: rounds (tiles over CUs, rounded up) times what
+// a round costs, a fixed part (first loads, last stores) and one per 32 elements
+// of K; where several small tiles share a CU, per tile. The estimate only has to
+// order the kernels near the lines between them; measured / estimated, graph-
+// replayed, the kernel taken first:
+//   4096^3 w 667 / 669, n 679 / 708; 1024 x 1024 x 128, batch 32 w 73 / 73, n 89 / 86
+//   2048^3 n 90 / 91, s 132 / 127; 1000 x 4096 x 1024 n 54 / 48, s 71 / 66
+//   2100 x 1900 x 170 n 21.2 / 13.4, s 21.4 / 16.4
+//   1024^3 s2 21.2 / 22.0, s 24.6 / 25.2; 970 x 1000 x 673 s2 18.1 / 16.0, s 19.3 / 18.2
+//   1000 x 1111 x 777 (B transposed) s 27.7 / 28.0, n 36 / 39, s2 38 / 36
+//   300 x 517 x 4096 ks 29.6 / 32.4, k16 41 / 42; 600 x 600 x 1000 ks 18.8 / 19.2,
+//   k16 20.9 / 26.5, s2 21.7 / 22.0; 512^3 ks 7.3 / 5.8, k16 10.9 / 11.8; 31 x 4096
+//   x 4096 ks 33.9 / 32.4, k16 34.0 / 35.0
+//   8 x 11008 x 4096 k16 41 / 46, ks 49 / 65; 16 x 4096 x 4096 k16 17.3 / 18.6, ks
+//   24 / 32; 256^3 k16 3.5 / 3.6, ks 4.8 / 3.9; 96 x 64 x 3776 k16 11.4 / 17.4, ks
+//   23 / 31
+// (ks is estimated from rounds that fill the card, and is up to a third faster
+// in the first; those shapes are k16's.) tiles(tm, tn): tiles of that size.
 template <class Tiles>
-static int plan_gemm_bf(vx_ctx ctx, uint32_t K, const Tiles& tiles, uint32_t pin) {
-    const double S = std::ceil(K / 32.0), cus = (double)ctx->num_cus;
+static int plan_gemm_bf(int num_cus, uint32_t K, const Tiles& tiles, uint32_t pin) {
+    const double S = std::ceil(K / 32.0), cus = (double)num_cus;
     double us[6];
     for (int i = 0; i < 6; ++i) {
         const double t = (double)tiles(kBfRows[i], kBfCols[i]) / cus, r = std::ceil(t);
@@ -473,7 +480,7 @@ static int run_gemm(vx_ctx ctx, vx_stream stream, const vx_mview* out, const vx_
     // Few outputs: 32 x 32 tiles with K split over a workgroup's waves, where
     // that is estimated fastest. This and the next choice come before the
     // pinned tile shape, so that all pins give the same bits at any shape.
-    const int cfg = plan_gemm_bf(ctx, p.K, tiles, pin);
+    const int cfg = plan_gemm_bf(ctx->num_cus, p.K, tiles, pin);
     // A short K and not many outputs, rows contiguous and 16-byte aligned: the
     // f32 MFMA kernels, whose tiles cost less to begin and to end (128 x 128 x
     // 128, batch 32: 7.4 against 7.9 us; 2432 x 2368 x 96 20.1 / 21.0; 200 x
@@ -868,11 +875,11 @@ static bool gemm_q_ok(const vx_qweight* w) { return xq_layout_ok(w) && w->cols <
 
 // The kernel (index into kGemmQ's last dimension) for M x K times B columns
 // with nt terms, and its estimated time.
-static int gemm_q_choose(vx_ctx ctx, uint32_t qt, uint32_t M, uint32_t K, uint32_t B, int nt, double* us) {
+static int gemm_q_choose(int num_cus, uint32_t qt, uint32_t M, uint32_t K, uint32_t B, int nt, double* us) {
     int best = 0;
     for (int c = 0; c < 4; ++c) {
         const double wgs = std::ceil((double)M / kGemmQRows[c]) * std::ceil((double)B / kGemmQCols[c]);
-        const double t = std::ceil(wgs / ctx->num_cus) * (K / 32u) * kGemmQ[nt - 2][qt == VX_Q8_0][c] * 1e-3;
+        const double t = std::ceil(wgs / num_cus) * (K / 32u) * kGemmQ[nt - 2][qt == VX_Q8_0][c] * 1e-3;
         if (c == 0 || t < *us) best = c, *us = t;
     }
     return best;
@@ -1024,7 +1031,7 @@ static int run_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y, const vx_
             // W streams once per tile of columns instead of once per 16 (a
             // caller that names the int8 split gets it)
             double us = 0.0;
-            const int cfg = gemm_q_choose(ctx, w->qtype, M, K, B, 2, &us);
+            const int cfg = gemm_q_choose(ctx->num_cus, w->qtype, M, K, B, 2, &us);
             if (us < gemv_xq_us(w->qtype, M, K, B)) return launch_gemm_q(ctx, stream, cy, w, cx, B, 2, cfg);
         }
         if (q.base) {
@@ -1040,7 +1047,7 @@ static int run_gemv_q(vx_ctx ctx, vx_stream stream, const vx_mview* y, const vx_
         // 4 8.3 against 10.6 us, 16448 x 4096 37 against 30; B = 8 17.3 / 10.7
         // and 78 / 31 us).
         double us = 0.0;
-        const int cfg = gemm_q_choose(ctx, w->qtype, M, K, B, 3, &us);
+        const int cfg = gemm_q_choose(ctx->num_cus, w->qtype, M, K, B, 3, &us);
         return launch_gemm_q(ctx, stream, cy, w, cx, B, 3, cfg);
     }
     // batch-1 kernel: the persistent one, or the per-row-group one when x
@@ -1511,6 +1518,17 @@ int vx_layout_unsqueeze(const vx_layout* in, uint32_t axis, vx_layout* out) {
     return vx::layout_unsqueeze(in, axis, out);
 }
 int vx_layout_is_contiguous(const vx_layout* in) { return in && vx::layout_is_contiguous(in) ? 1 : 0; }
+
+int vx_plan_gemm_bf(int num_cus, uint32_t M, uint32_t N, uint32_t K, uint32_t batch, uint32_t pin) {
+    return vx::plan_gemm_bf(num_cus, K, [&](uint32_t tm, uint32_t tn) {
+        return (uint64_t)((M + (uint64_t)tm - 1) / tm) * ((N + (uint64_t)tn - 1) / tn) * batch;
+    }, pin);
+}
+int vx_plan_gemm_q(int num_cus, uint32_t qtype, uint32_t M, uint32_t K, uint32_t B, int terms) {
+    double us = 0.0;
+    const int cfg = vx::gemm_q_choose(num_cus, qtype, M, K, B, terms, &us);
+    return terms == 2 && !(us < vx::gemv_xq_us(qtype, M, K, B)) ? -1 : cfg;
+}
 
 const char* vx_status_string(int status) {
     switch (status) {

@@ -26,3 +26,11 @@ int layout_narrow(const vx_layout* in, uint32_t axis, uint32_t first, uint32_t c
 int layout_unsqueeze(const vx_layout* in, uint32_t axis, vx_layout* out);
 
 }  // namespace vx
+
+// Which kernel a shape takes on a device of num_cus CUs, for the tests (they
+// check that their shapes reach every one). GEMM on bf16 terms: 0..5 for w, n,
+// s2, s, ks, k16 (see plan_gemm_bf). Quantized product with many columns of x in
+// two or three terms: 0..3 for 32 x 16, 64 x 16, 64 x 32 with K split, 256 x 128;
+// -1 where two terms lose to the int8 split.
+extern "C" int vx_plan_gemm_bf(int num_cus, uint32_t M, uint32_t N, uint32_t K, uint32_t batch, uint32_t pin);
+extern "C" int vx_plan_gemm_q(int num_cus, uint32_t qtype, uint32_t M, uint32_t K, uint32_t B, int terms);
