@@ -101,24 +101,30 @@ struct vx_slab {
 };
 
 // One operand's chunk of 32 elements of K of lane (n, g)'s x for the bf16 terms:
-// H pieces of 8 elements (H G = 4; 32 x 32 tiles: g 0..1; 16 x 16: g 0..3).
-template <int MODE, int H, int G>
+// H pieces of 8 elements (H G = 4; 32 x 32 tiles: g 0..1; 16 x 16: g 0..3). SO:
+// the lane group's part of the address in the base, the rest a scalar offset,
+// where both operands are read along M / N (600 x 600 x 1000 17.6 -> 16.9 us; with
+// one along K the lane's offset in every address is as fast or faster, 300 x 517 x
+// 600 7.11 / 6.99).
+template <int MODE, int H, int G, bool SO>
 struct vx_chunk {
     static constexpr uint32_t KC = 8u * G * H;
     float r[H][8];
-    // where the lane's pieces of chunk 0 begin in its row or column p
-    static __device__ __forceinline__ const float* base(const float* p, int64_t sk, uint32_t g) { return p + (int64_t)(8u * g) * sk; }
-    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0) {
+    // what load and load_tail take for the lane's row or column p
+    static __device__ __forceinline__ const float* base(const float* p, int64_t sk, uint32_t g) {
+        return SO ? p + (int64_t)(8u * g) * sk : p;
+    }
+    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0, uint32_t g) {
 #pragma unroll
         for (int h = 0; h < H; ++h) {
             if constexpr (MODE == MODE_K) {
-                const float* q = p + (k0 + 8u * G * h);
+                const float* q = p + (k0 + 8u * G * h + 8u * g);
                 const f32x4_a4 a = *(const f32x4_a4*)q, b = *(const f32x4_a4*)(q + 4);
                 r[h][0] = a.x; r[h][1] = a.y; r[h][2] = a.z; r[h][3] = a.w;
                 r[h][4] = b.x; r[h][5] = b.y; r[h][6] = b.z; r[h][7] = b.w;
             } else {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) r[h][j] = p[(int64_t)(k0 + 8u * G * h + (uint32_t)j) * sk];  // (a scalar offset)
+                for (int j = 0; j < 8; ++j) r[h][j] = p[(int64_t)(k0 + 8u * G * h + (SO ? 0u : 8u * g) + (uint32_t)j) * sk];
             }
         }
     }
@@ -128,7 +134,7 @@ struct vx_chunk {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const uint32_t k = k0 + 8u * G * h + 8u * g + (uint32_t)j, kc = min(k, K - 1u);
-                const float e = p[((int64_t)kc - 8u * g) * (MODE == MODE_K ? 1 : sk)];  // (clamped: no branches between the loads)
+                const float e = MODE == MODE_K ? p[kc] : p[((int64_t)kc - (SO ? 8u * g : 0u)) * sk];  // (clamped: no branches between the loads)
                 r[h][j] = k < K ? e : 0.f;
             }
     }
@@ -142,7 +148,7 @@ struct vx_seq {
     static constexpr int NS = 16 / G, NR = MODE == MODE_K ? 16 : NS;
     float r[NR];
     static __device__ __forceinline__ const float* base(const float* p, int64_t sk, uint32_t g) { return MODE == MODE_K ? p : p + (int64_t)g * sk; }
-    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0) {
+    __device__ __forceinline__ void load(const float* p, int64_t sk, uint32_t k0, uint32_t) {
         if constexpr (MODE == MODE_K) {
 #pragma unroll
             for (int j = 0; j < 16; j += 4) {
@@ -193,8 +199,8 @@ __device__ __forceinline__ void vx_chunks(const vx_gemm_args& p, const float* pa
         CB b[2];
         const uint32_t last = (nck - 1u - w) / nw * nw + w;  // this wave's last chunk
         auto load = [&](int d, uint32_t c) {
-            a[d].load(pa, p.as[3], min(c, last) * KC);
-            b[d].load(pb, p.bs[2], min(c, last) * KC);
+            a[d].load(pa, p.as[3], min(c, last) * KC, g);
+            b[d].load(pb, p.bs[2], min(c, last) * KC, g);
         };
         load(0, w);
         load(1, w + nw);
@@ -562,7 +568,8 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
                                                                  __builtin_bit_cast(bf16x8, tb[TB[e]]), acc[h], 0, 0, 0);
         }
     };
-    vx_chunks<vx_chunk<AM, 2, 2>, vx_chunk<BM, 2, 2>>(p, pa, pb, g, wave, NWV, mult);
+    constexpr bool SO = AM == MODE_X && BM == MODE_X;
+    vx_chunks<vx_chunk<AM, 2, 2, SO>, vx_chunk<BM, 2, 2, SO>>(p, pa, pb, g, wave, NWV, mult);
     // red[wave][v][lane], and whether the tile needs a closer look
     float* red = (float*)vx_bf_lds;
     uint32_t* word = (uint32_t*)(red + NWV * 1024u);
@@ -658,7 +665,8 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
             acc[par] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ta[TA[e]]),
                                                                __builtin_bit_cast(bf16x8, tb[TB[e]]), acc[par], 0, 0, 0);
     };
-    vx_chunks<vx_chunk<AM, 1, 4>, vx_chunk<BM, 1, 4>>(p, pa, pb, g, wave, NWV, mult);
+    constexpr bool SO = AM == MODE_X && BM == MODE_X;
+    vx_chunks<vx_chunk<AM, 1, 4, SO>, vx_chunk<BM, 1, 4, SO>>(p, pa, pb, g, wave, NWV, mult);
     // red[wave][v][lane], and whether the tile needs a closer look
     float* red = (float*)vx_bf_lds;
     uint32_t* word = (uint32_t*)(red + NWV * 256u);
