@@ -9,11 +9,12 @@
 // at K = 4096 7.1e-7 off 64 bits against 1.15e-6, with fewer additions in
 // f32), at six times the MFMA work but sixteen times the rate.
 //
-// Measured (graph-replayed, same box, against the f32 MFMA kernels): 4096^3 980
-// -> 650 us (212 TFLOP/s of f32 work, 1270 of bf16; a bf16 product of that size
-// by the vendor's library 1370 on this card), 4096 x 11008 x 4096 2720 -> 1870,
-// 1024^3 26 -> 23.5, 1000 x 1111 x 777 with odd strides 119 -> 28, 8 x 11008 x
-// 4096 154 -> 44 (K split), 64 x 64 x 4096 394 -> 13 (K split). The large
+// Measured (graph-replayed with the same operands, same box, against the f32 MFMA
+// kernels): 4096^3 973 -> 647 us (212 TFLOP/s of f32 work, 1275 of bf16; a bf16
+// product of that size by the vendor's library 1370 on this card), 4096 x 11008 x
+// 4096 2698 -> 1813, 1024^3 22.7 -> 19.3, 1000 x 1111 x 777 with odd strides 119
+// -> 26.8, 8 x 11008 x 4096 150 -> 41 (K split; with new operands each call 179 ->
+// 44), 64 x 64 x 4096 392 -> 12 (K split). The large
 // shapes are bound by the matrix cores and the card's power, the smaller ones
 // by the stages' serial steps (load, convert, store, barrier, read, multiply)
 // with one workgroup per CU.
@@ -586,58 +587,62 @@ __device__ __forceinline__ void vx_gemm_bf_ks(const vx_gemm_args& p) {
     }
     if ((lost & 0xFFFFu) != 0u || vx_gemm_bf_odd(s[0]) || vx_gemm_bf_odd(s[1])) *word = 1u;
     __syncthreads();
-    const bool look = *word != 0u;
-    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + 64;  // of each row of A and column of B, see vx_scan
-    if (look) {
-        if (t < 128u) mx[t] = 0u;
-        __syncthreads();
-        auto all = [](uint32_t) { return true; };
-        vx_scan<AM == MODE_K, 32>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NWV, lane, mx, ls, all);
-        vx_scan<BM == MODE_K, 32>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 32, ls + 32, all);
-        __syncthreads();
-    }
-    bool again[2] = {false, false};  // outputs to form from f32 products
     const uint32_t rt0 = 8u * (t >> 8) + 4u * (lane >> 5) + (wave & 3u), ct = lane & 31u;  // output u: row rt0 + 16 u, column ct
-    if (look) {
+    auto write = [&] {
+#pragma unroll
+        for (uint32_t u = 0; u < 2u; ++u) {
+            const uint32_t row = m0 + rt0 + 16u * u, col = n0 + ct;
+            if (row < p.M && col < p.N) vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s[u], p.alpha, p.beta);
+        }
+    };
+    // (the usual end first and by itself: with the look between, 512^3 took 7.4
+    // us instead of 7.2, 600 x 600 x 1000 17.6 instead of 17.2)
+    if (__builtin_expect(*word == 0u, 1)) {
+        write();
+        return;
+    }
+    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + 64;  // of each row of A and column of B, see vx_scan
+    if (t < 128u) mx[t] = 0u;
+    __syncthreads();
+    auto all = [](uint32_t) { return true; };
+    vx_scan<AM == MODE_K, 32>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NWV, lane, mx, ls, all);
+    vx_scan<BM == MODE_K, 32>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 32, ls + 32, all);
+    __syncthreads();
+    bool again[2];  // outputs to form from f32 products
+#pragma unroll
+    for (uint32_t u = 0; u < 2u; ++u)
+        again[u] = vx_gemm_bf_again(s[u], p.K, mx[rt0 + 16u * u], ls[rt0 + 16u * u] != 0u, mx[32u + ct], ls[32u + ct] != 0u);
+    if (again[0] || again[1]) *word = 2u;
+    __syncthreads();
+    if (*word == 2u) {
+        if (wave < 4u) {  // 16 x 16 outputs each
+            const uint32_t r0 = 16u * (wave >> 1), c0 = 16u * (wave & 1u), n16 = lane & 15u, g4 = lane >> 4;
+            f32x4 f;
+            vx_f32_tile<AM, BM>(p, A + (int64_t)min(m0 + r0 + n16, p.M - 1u) * p.as[2],
+                                B + (int64_t)min(n0 + c0 + n16, p.N - 1u) * p.bs[3], g4, f);
+#pragma unroll
+            for (uint32_t v = 0; v < 4u; ++v) red[(r0 + 4u * g4 + v) * 32u + c0 + n16] = f[v];
+        }
+        __syncthreads();
 #pragma unroll
         for (uint32_t u = 0; u < 2u; ++u)
-            again[u] = vx_gemm_bf_again(s[u], p.K, mx[rt0 + 16u * u], ls[rt0 + 16u * u] != 0u, mx[32u + ct], ls[32u + ct] != 0u);
-        if (again[0] || again[1]) *word = 2u;
-        __syncthreads();
-        if (*word == 2u) {
-            if (wave < 4u) {  // 16 x 16 outputs each
-                const uint32_t r0 = 16u * (wave >> 1), c0 = 16u * (wave & 1u), n16 = lane & 15u, g4 = lane >> 4;
-                f32x4 f;
-                vx_f32_tile<AM, BM>(p, A + (int64_t)min(m0 + r0 + n16, p.M - 1u) * p.as[2],
-                                    B + (int64_t)min(n0 + c0 + n16, p.N - 1u) * p.bs[3], g4, f);
-#pragma unroll
-                for (uint32_t v = 0; v < 4u; ++v) red[(r0 + 4u * g4 + v) * 32u + c0 + n16] = f[v];
-            }
-            __syncthreads();
-#pragma unroll
-            for (uint32_t u = 0; u < 2u; ++u)
-                if (again[u]) s[u] = red[(rt0 + 16u * u) * 32u + ct];
-        }
+            if (again[u]) s[u] = red[(rt0 + 16u * u) * 32u + ct];
     }
-#pragma unroll
-    for (uint32_t u = 0; u < 2u; ++u) {
-        const uint32_t row = m0 + rt0 + 16u * u, col = n0 + ct;
-        if (row < p.M && col < p.N) vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s[u], p.alpha, p.beta);
-    }
+    write();
 }
 
 // 16 x 16 tiles on 16 x 16 x 32 products, K split over the 8 waves as above.
 // Against 32 x 32 tiles, four times the workgroups, and few enough registers
-// for two or three on a CU: the shapes with about as many 32 x 32 tiles as CUs,
+// for two on a CU: the shapes with about as many 32 x 32 tiles as CUs,
 // or fewer, ran at the pace of one workgroup on some of the CUs (or of a second
 // round on a few). Each operand is read and split once per 16 outputs of the
 // other, so it loses where 32 x 32 tiles fill the card. Graph-replayed, us, 32 x
-// 32 / 16 x 16: 8 x 11008 x 4096 B [N, K] 52.7 / 44.1, 16 x 4096 x 4096 28.4 /
-// 19.5, 23 x 1989 x 5973 34.8 / 22.0, 96 x 64 x 3776 A [K, M] 24.9 / 13.1, 256^3
-// 5.3 / 4.1; but 30 x 16384 x 2048 41 / 73, 512^3 8.0 / 12.2. Tried: 4 or 16
-// waves (44.4, 47.2 us on the first), three or four chunks ahead (no gain), 32 x
-// 16 tiles (46.3; 31 x 4096 x 4096 25.6 against 33.7 and 34.5, the only size
-// where they won).
+// 32 / 16 x 16: 8 x 11008 x 4096 B [N, K] 49.4 / 41.0, 16 x 4096 x 4096 24.2 /
+// 17.3, 23 x 1989 x 5973 34.6 / 22.4, 96 x 64 x 3776 23.4 / 11.4, 256^3 4.8 / 3.5;
+// but 30 x 16384 x 2048 38.7 / 72.4, 512^3 7.3 / 10.9. Tried, when the first of
+// these took 44.1 us: 4 or 16 waves (44.4, 47.2), three or four chunks ahead (no
+// gain), 32 x 16 tiles (46.3; 31 x 4096 x 4096 25.6 against 33.7 and 34.5, the
+// only size where they won).
 template <int AM, int BM>
 __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
     constexpr uint32_t NWV = 8;
@@ -679,34 +684,36 @@ __device__ __forceinline__ void vx_gemm_bf_k16(const vx_gemm_args& p) {
     for (uint32_t w = 1; w < NWV; ++w) s += red[w * 256u + (t & 255u)];
     if ((lost & 0xFFFFu) != 0u || vx_gemm_bf_odd(s)) *word = 1u;
     __syncthreads();
-    const bool look = *word != 0u;
-    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + 32;  // of each row of A and column of B, see vx_scan
-    if (look) {
-        if (t < 64u) mx[t] = 0u;
-        __syncthreads();
-        auto all = [](uint32_t) { return true; };
-        vx_scan<AM == MODE_K, 16>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NWV, lane, mx, ls, all);
-        vx_scan<BM == MODE_K, 16>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 16, ls + 16, all);
-        __syncthreads();
-    }
     const uint32_t rt = 4u * (lane >> 4) + (wave & 3u), ct = lane & 15u;  // of the first four waves' outputs
-    if (look) {
-        const bool again = vx_gemm_bf_again(s, p.K, mx[rt], ls[rt] != 0u, mx[16u + ct], ls[16u + ct] != 0u);
-        if (again) *word = 2u;
-        __syncthreads();
-        if (*word == 2u) {
-            if (wave == 0u) {
-                f32x4 f;
-                vx_f32_tile<AM, BM>(p, pa, pb, g, f);
-#pragma unroll
-                for (uint32_t v = 0; v < 4u; ++v) red[v * 64u + lane] = f[v];
-            }
-            __syncthreads();
-            if (again) s = red[t & 255u];
-        }
+    auto write = [&] {
+        const uint32_t row = m0 + rt, col = n0 + ct;
+        if (t < 256u && row < p.M && col < p.N) vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+    };
+    if (__builtin_expect(*word == 0u, 1)) {  // (as in vx_gemm_bf_ks)
+        write();
+        return;
     }
-    const uint32_t row = m0 + rt, col = n0 + ct;
-    if (t < 256u && row < p.M && col < p.N) vx_epilogue(C + (int64_t)row * p.cs[2] + (int64_t)col * p.cs[3], s, p.alpha, p.beta);
+    uint32_t *mx = (uint32_t*)vx_bf_lds, *ls = mx + 32;  // of each row of A and column of B, see vx_scan
+    if (t < 64u) mx[t] = 0u;
+    __syncthreads();
+    auto all = [](uint32_t) { return true; };
+    vx_scan<AM == MODE_K, 16>(A, p.as[2], p.as[3], m0, p.M, p.K, wave, NWV, lane, mx, ls, all);
+    vx_scan<BM == MODE_K, 16>(B, p.bs[3], p.bs[2], n0, p.N, p.K, wave, NWV, lane, mx + 16, ls + 16, all);
+    __syncthreads();
+    const bool again = vx_gemm_bf_again(s, p.K, mx[rt], ls[rt] != 0u, mx[16u + ct], ls[16u + ct] != 0u);
+    if (again) *word = 2u;
+    __syncthreads();
+    if (*word == 2u) {
+        if (wave == 0u) {
+            f32x4 f;
+            vx_f32_tile<AM, BM>(p, pa, pb, g, f);
+#pragma unroll
+            for (uint32_t v = 0; v < 4u; ++v) red[v * 64u + lane] = f[v];
+        }
+        __syncthreads();
+        if (again) s = red[t & 255u];
+    }
+    write();
 }
 
 // 256 x 128 tiles (8 waves of 64 x 64), 128 x 128 (2 x 4 waves of 64 x 64) and
