@@ -704,7 +704,7 @@ def roof(r: dict, key: str, bound: str = "hbm") -> dict:
         a, peak, unit = r["alg_bytes"] / t / 1e9, HBM_PEAK_GBS, "GB/s"
     else:
         a, peak, unit = r["flops"] / t / 1e12, rnd(GEMM_PEAK_TFS), "TFLOP/s"
-    tr = load_traffic(key) if bound == "hbm" else None  # (the GEMM's counter runs are of its former kernels)
+    tr = load_traffic(key)
     return {"bound": bound, "achieved": rnd(a), "peak": peak, "unit": unit, "frac": rnd(a / peak, 3),
             "traffic": int(tr) if tr else None}
 
@@ -805,6 +805,8 @@ def main() -> int:
                                                                                floor["step_ms_events"]) * 1e-3) / 1e9)},
         "gemm_4096": dict(gline("gemm_f32_4096", GEMMS["gemm_f32_4096"][4], "TFLOP/s", "mfma"),
                           steps=GEMM_STEPS, warmup=GEMM_WARMUP,
+                          arithmetic="f32 operands as three bf16 terms each, six bf16 products per f32 product, f32 sums; "
+                                     "peak = dense bf16 2516.6 / 6",
                           cpu_baseline=cpu["gemm4096"] if cpu else None),
         # compact lines: key -> [value, ms per step, roofline achieved, roofline frac, launches per step]
         "lines_fields": ["value", "ms_per_step", "roof_achieved", "roof_frac", "launches"],
